@@ -13,9 +13,11 @@
 // kernel of an iteration first reads a device stop flag and returns when it is
 // set, so the host queues a block of iterations at a time and reads the flag
 // once per block.  Dot products are fused into the producing kernels as
-// per-workgroup partials and reduced by one workgroup per segment in a fixed
-// order: results are deterministic and independent of what else runs on the
-// GPU.  With opt.graph the block of iterations is captured once into a HIP
+// per-workgroup partials and reduced in a fixed order, by one workgroup per
+// segment or, where no segment has more than kFusedParts partials, by every
+// workgroup of the kernel that needs the sum (the same order and bits, two
+// launches fewer an iteration): results are deterministic and independent of
+// what else runs on the GPU.  With opt.graph the block of iterations is captured once into a HIP
 // graph and replayed (the kernels and their order are unchanged, so the
 // results are bit-identical to the eager launches).
 //
@@ -49,9 +51,7 @@ __global__ __launch_bounds__(256) void k_rhs_tod(const double *__restrict__ s, c
     if (t < m) tod[t] = (s[t] + n[t]) - 0.0;
 }
 
-__global__ __launch_bounds__(256) void k_map_to_f32(const double *__restrict__ a, float *__restrict__ b, int n,
-                                                    const int *__restrict__ flag) {
-    if (flag && stopped(flag)) return;
+__global__ __launch_bounds__(256) void k_map_to_f32(const double *__restrict__ a, float *__restrict__ b, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) b[i] = (float) a[i];
 }
@@ -134,22 +134,39 @@ __global__ __launch_bounds__(kRB) void k_coeff(const double *__restrict__ part, 
     }
 }
 
+// ro = g2pix / coeff: k_coeff's S_RO, or (FUSED) coeff summed here from the
+// partials of <h,q> and g2pix from the slot `cur` of this iteration
+template <bool FUSED>
+__device__ __forceinline__ double step_length(const double *__restrict__ S, int r, const double *__restrict__ dot,
+                                              const int *__restrict__ wg0, int cur, double *red) {
+    const double *Sr = S + (int64_t) r * S_NSCAL;
+    if constexpr (FUSED) {
+        double coeff[1];
+        reduce_parts_wg<1>(dot + wg0[r], 0, wg0[r + 1] - wg0[r], red, coeff);
+        return Sr[cur] / coeff[0];
+    } else {
+        return Sr[S_RO];
+    }
+}
+
 // x += ro h; g = gp - ro q; Cg = M g; partials <Cg,g>, <Cg,g-gp>, <g,g>
+template <bool FUSED>
 __global__ __launch_bounds__(kMB) void k_update(double *__restrict__ x, const double *__restrict__ h,
                                                 double *__restrict__ g, const double *__restrict__ gp,
                                                 const double *__restrict__ qv, const double *__restrict__ inv,
                                                 double *__restrict__ Cg, const int *__restrict__ wg_seg,
                                                 const int *__restrict__ wg_q0, const int *__restrict__ seg_q,
                                                 const double *__restrict__ S, const int *__restrict__ state,
-                                                double *__restrict__ part, const int *__restrict__ flag) {
+                                                double *__restrict__ part, const int *__restrict__ flag,
+                                                const double *__restrict__ dot, const int *__restrict__ wg0, int cur) {
     if (stopped(flag)) return;
     const SegPix sp = seg_pixel(wg_seg, wg_q0, seg_q);
     if (state[sp.r]) return;  // frozen segment (uniform over the workgroup)
-    __shared__ double red[kMB / 64];
+    __shared__ double red[FUSED ? kRB / 64 : kMB / 64];
     const int q = sp.q;
+    const double ro = step_length<FUSED>(S, sp.r, dot, wg0, cur, red);
     double a = 0.0, b = 0.0, c = 0.0;
     if (q < sp.qend) {
-        const double ro = S[(int64_t) sp.r * S_NSCAL + S_RO];
         double gn[3], gpv[3];
         for (int r = 0; r < 3; r++) {
             const int i = 3 * q + r;
@@ -181,16 +198,20 @@ __global__ __launch_bounds__(kMB) void k_update(double *__restrict__ x, const do
 }
 
 // x += ro h; g = gp - ro q (the two-level preconditioner applies M and the dots afterwards)
+template <bool FUSED>
 __global__ __launch_bounds__(kMB) void k_update_xg(double *__restrict__ x, const double *__restrict__ h,
                                                    double *__restrict__ g, const double *__restrict__ gp,
                                                    const double *__restrict__ qv, const int *__restrict__ wg_seg,
                                                    const int *__restrict__ wg_q0, const int *__restrict__ seg_q,
                                                    const double *__restrict__ S, const int *__restrict__ state,
-                                                   const int *__restrict__ flag) {
+                                                   const int *__restrict__ flag, const double *__restrict__ dot,
+                                                   const int *__restrict__ wg0, int cur) {
     if (stopped(flag)) return;
     const SegPix sp = seg_pixel(wg_seg, wg_q0, seg_q);
-    if (state[sp.r] || sp.q >= sp.qend) return;
-    const double ro = S[(int64_t) sp.r * S_NSCAL + S_RO];
+    if (state[sp.r]) return;
+    __shared__ double red[kRB / 64];
+    const double ro = step_length<FUSED>(S, sp.r, dot, wg0, cur, red);
+    if (sp.q >= sp.qend) return;
     for (int r = 0; r < 3; r++) {
         const int i = 3 * sp.q + r;
         x[i] = x[i] + ro * h[i];
@@ -198,13 +219,56 @@ __global__ __launch_bounds__(kMB) void k_update_xg(double *__restrict__ x, const
     }
 }
 
-// dots -> g2pix, polak, res; history; stop test; gamma.  One workgroup per segment.
+// The scalars of segment r after an iteration, by one thread: g2pix, polak, res
+// recorded; history; stop test; returns gamma.  The g2pix of the iteration is
+// in slot `cur` and the new one goes to slot `nxt` (the two alternate, so that
+// the other workgroups of a fused kernel still read the old one).
 // kind (IT_*): where a segment's g was updated in FP32 this iteration (mixed
 // precision, the segment not refreshed), a passing stop test does not stop it:
 // it sets S_PEND (counted in F_NPEND) and the first iteration of the next block
 // refreshes that segment's residual in FP64, whose test decides.  Whether a
 // segment refreshes depends on its own state and the iteration number only,
 // so a segment runs the same iterations alone and in a batch.
+__device__ __forceinline__ void segment_scalars(double *__restrict__ Sr, int r, double g2pix, double polak, double res,
+                                                int nxt, double *__restrict__ hist, int maxiter,
+                                                int *__restrict__ state, int nseg, int *__restrict__ flag, int kind,
+                                                int adaptive) {
+    const double k = Sr[S_K] + 1.0;
+    Sr[S_K] = k;
+    Sr[nxt] = g2pix;
+    Sr[S_POLAK] = polak;
+    Sr[S_RES] = res;
+    const int ki = (int) k;
+    if (hist && ki < maxiter) hist[(int64_t) r * maxiter + ki] = sqrt(res) / sqrt(Sr[S_RES0]);
+    atomicMax(&flag[F_KMAX], ki);
+    const bool pend = Sr[S_PEND] != 0.0;
+    const bool refreshed = kind == IT_REFRESH_ALL || (kind == IT_REFRESH_PENDING && pend);
+    const bool verify = kind != IT_FP64 && !refreshed;
+    bool pend_now = pend && !refreshed;
+    if (refreshed) {
+        Sr[S_RREF] = res;
+        Sr[S_KREF] = k;
+    }
+    int st = 0;
+    if (res <= Sr[S_TOL2] && !verify)
+        st = 1;
+    else if ((Sr[S_STOPK] > 0.0 && k >= Sr[S_STOPK]) || k + 1.0 >= Sr[S_MAXK])
+        st = 2;
+    if (res <= Sr[S_TOL2] && verify) pend_now = true;
+    if (adaptive && verify && (res <= kAdaptDrop * Sr[S_RREF] || k - Sr[S_KREF] >= kAdaptGap)) pend_now = true;
+    if (st) pend_now = false;
+    if (pend_now != pend) {
+        Sr[S_PEND] = pend_now ? 1.0 : 0.0;
+        atomicAdd(&flag[F_NPEND], pend_now ? 1 : -1);
+    }
+    if (st) {
+        state[r] = st;
+        if (r == 0 && st == 1) flag[F_CONV0] = 1;
+        segment_done(flag, nseg);
+    }
+}
+
+// dots -> the segment's scalars and gamma.  One workgroup per segment.
 __global__ __launch_bounds__(kRB) void k_scalars(const double *__restrict__ part, int nwg,
                                                  const int *__restrict__ wg0, double *__restrict__ S,
                                                  double *__restrict__ hist, int maxiter, int *__restrict__ state,
@@ -221,56 +285,50 @@ __global__ __launch_bounds__(kRB) void k_scalars(const double *__restrict__ part
     const double res = reduce_parts(part + 2 * nwg + p0, np, red);
     if (threadIdx.x == 0) {
         double *Sr = S + (int64_t) r * S_NSCAL;
-        const double k = Sr[S_K] + 1.0;
-        Sr[S_K] = k;
-        Sr[S_G2PIXP] = Sr[S_G2PIX];
-        Sr[S_G2PIX] = g2pix;
-        Sr[S_POLAK] = polak;
-        Sr[S_RES] = res;
-        const int ki = (int) k;
-        if (hist && ki < maxiter) hist[(int64_t) r * maxiter + ki] = sqrt(res) / sqrt(Sr[S_RES0]);
-        atomicMax(&flag[F_KMAX], ki);
-        const bool pend = Sr[S_PEND] != 0.0;
-        const bool refreshed = kind == IT_REFRESH_ALL || (kind == IT_REFRESH_PENDING && pend);
-        const bool verify = kind != IT_FP64 && !refreshed;
-        bool pend_now = pend && !refreshed;
-        if (refreshed) {
-            Sr[S_RREF] = res;
-            Sr[S_KREF] = k;
-        }
-        int st = 0;
-        if (res <= Sr[S_TOL2] && !verify)
-            st = 1;
-        else if ((Sr[S_STOPK] > 0.0 && k >= Sr[S_STOPK]) || k + 1.0 >= Sr[S_MAXK])
-            st = 2;
-        if (res <= Sr[S_TOL2] && verify) pend_now = true;
-        if (adaptive && verify && (res <= kAdaptDrop * Sr[S_RREF] || k - Sr[S_KREF] >= kAdaptGap)) pend_now = true;
-        if (st) pend_now = false;
-        if (pend_now != pend) {
-            Sr[S_PEND] = pend_now ? 1.0 : 0.0;
-            atomicAdd(&flag[F_NPEND], pend_now ? 1 : -1);
-        }
-        if (st) {
-            state[r] = st;
-            if (r == 0 && st == 1) flag[F_CONV0] = 1;
-            segment_done(flag, nseg);
-        }
-        Sr[S_GAMMA] = polak / Sr[S_G2PIXP];
+        Sr[S_GAMMA] = polak / Sr[S_G2PIX];
+        segment_scalars(Sr, r, g2pix, polak, res, S_G2PIX, hist, maxiter, state, nseg, flag, kind, adaptive);
     }
 }
 
-// h = h gamma + Cg
+// h = h gamma + Cg, and its FP32 copy where the next product is in FP32.
+// FUSED: every workgroup sums its segment's three dots itself; the first
+// workgroup of a segment then does k_scalars' work.  It may stop the segment
+// (or the solve) while the others still run: they skip or finish an h that
+// nothing reads any more, but each decides once for all its threads.
+template <bool FUSED>
 __global__ __launch_bounds__(kMB) void k_hupdate(double *__restrict__ h, const double *__restrict__ Cg,
-                                                 const int *__restrict__ wg_seg, const int *__restrict__ wg_q0,
-                                                 const int *__restrict__ seg_q, const double *__restrict__ S,
-                                                 const int *__restrict__ state, const int *__restrict__ flag) {
-    if (stopped(flag)) return;
+                                                 float *__restrict__ hf, const int *__restrict__ wg_seg,
+                                                 const int *__restrict__ wg_q0, const int *__restrict__ seg_q,
+                                                 double *__restrict__ S, int *__restrict__ state,
+                                                 int *__restrict__ flag, const double *__restrict__ part, int nwg,
+                                                 const int *__restrict__ wg0, int cur, int nxt,
+                                                 double *__restrict__ hist, int maxiter, int nseg, int kind,
+                                                 int adaptive) {
     const SegPix sp = seg_pixel(wg_seg, wg_q0, seg_q);
-    if (state[sp.r] || sp.q >= sp.qend) return;
-    const double gamma = S[(int64_t) sp.r * S_NSCAL + S_GAMMA];
+    double gamma;
+    if constexpr (FUSED) {
+        __shared__ double red[3 * kRB / 64];
+        __shared__ int skip;
+        if (threadIdx.x == 0) skip = stopped(flag) || stopped(state + sp.r);
+        __syncthreads();
+        if (skip) return;
+        const int p0 = wg0[sp.r];
+        double *Sr = S + (int64_t) sp.r * S_NSCAL;
+        double dots[3];
+        reduce_parts_wg<3>(part + p0, nwg, wg0[sp.r + 1] - p0, red, dots);
+        gamma = dots[1] / Sr[cur];
+        if (threadIdx.x == 0 && (int) blockIdx.x == p0)
+            segment_scalars(Sr, sp.r, dots[0], dots[1], dots[2], nxt, hist, maxiter, state, nseg, flag, kind, adaptive);
+    } else {
+        if (stopped(flag) || state[sp.r]) return;
+        gamma = S[(int64_t) sp.r * S_NSCAL + S_GAMMA];
+    }
+    if (sp.q >= sp.qend) return;
     for (int c = 0; c < 3; c++) {
         const int i = 3 * sp.q + c;
-        h[i] = h[i] * gamma + Cg[i];
+        const double v = h[i] * gamma + Cg[i];
+        h[i] = v;
+        if (hf) hf[i] = (float) v;
     }
 }
 
@@ -553,8 +611,8 @@ int ensure_work(Problem &pb) {
     }
     if (!pb.d_map[0])
         for (int i = 0; i < 8; i++) MGPU_RET(pb.arena.alloc(&pb.d_map[i], (size_t) n0));
-    // partials: 3 per map workgroup (at most one extra workgroup per segment)
-    const int64_t need_red = 3 * ((int64_t) grid_for(pb.pt.npix0, kMB) + pb.sg.nseg + 1) + 64;
+    // partials: <h,q> and three dots per map workgroup (at most one extra workgroup per segment)
+    const int64_t need_red = 4 * ((int64_t) grid_for(pb.pt.npix0, kMB) + pb.sg.nseg + 1) + 64;
     if (pb.d_red && pb.nred < need_red) {
         pb.arena.release(pb.d_red);
         pb.d_red = nullptr;
@@ -598,11 +656,9 @@ int apply_A64(Problem &pb, const double *d_v, double *d_out, double *d_dot) {
     return MGPU_OK;
 }
 
-static int apply_A32(Problem &pb, const double *d_v, double *d_out, double *d_dot, const int *d_flag) {
-    const int n = 3 * pb.pt.npix;
+// q = A v in FP32 products; pb.d_mapf holds v's FP32 copy (k_hupdate writes it)
+static int apply_A32(Problem &pb, const double *d_v, double *d_out, double *d_dot) {
     pb.prof.begin(MGPU_KT_P, pb.stream);
-    k_map_to_f32<<<grid_for(n, 256), 256, 0, pb.stream>>>(d_v, pb.d_mapf, n, d_flag);
-    MGPU_LAUNCHED();
     MGPU_RET(launch_matvec_f32(pb, pb.d_mapf, pb.d_todf, true));
     pb.prof.end(pb.stream);
     MGPU_RET(toeplitz_apply_f32(pb, pb.d_todf, pb.d_tod2f, false));
@@ -654,6 +710,11 @@ int pcg_run(Problem &pb, const double *d_signal, const double *d_noise, double t
     int *flag = pb.d_flag;
     int *state = G.d_state;
     const int *wseg = G.d_wg_seg, *wq0 = G.d_wg_q0, *sq = G.d_q, *wg0 = G.d_wg0;
+    // the map kernels sum the dots' partials themselves where every segment has few (kFusedParts)
+    int most_parts = 0;
+    for (int r = 0; r < nseg; r++) most_parts = std::max(most_parts, G.h_wg0[r + 1] - G.h_wg0[r]);
+    const bool fused = most_parts <= kFusedParts;
+    double *dot = part + 3 * (int64_t) nwg;  // partials of <h,q>, read while k_update writes its own
     double *d_hist = nullptr;
     if (h_hist) {
         MGPU_RET(pb.arena.alloc(&d_hist, (size_t) maxiter * nseg));
@@ -702,6 +763,10 @@ int pcg_run(Problem &pb, const double *d_signal, const double *d_noise, double t
     }
     k_init_scalars<<<nseg, kRB, 0, s>>>(part, nwg, wg0, S, d_hist, maxiter, state, nseg, flag);
     MGPU_LAUNCHED();
+    if (mixed) {
+        k_map_to_f32<<<grid_for(n, 256), 256, 0, s>>>(h, pb.d_mapf, n);
+        MGPU_LAUNCHED();
+    }
 
     // from here on P, N^-1 and P^T skip the work of stopped segments (every
     // segment is computed again after the loop, for the true residual)
@@ -745,18 +810,26 @@ int pcg_run(Problem &pb, const double *d_signal, const double *d_noise, double t
         std::swap(g, gp);  // pcg_true.c:140-142
         // q = A h with fused <h, q>
         if (mixed)
-            MGPU_RET(apply_A32(pb, h, qv, part, flag));
+            MGPU_RET(apply_A32(pb, h, qv, dot));
         else
-            MGPU_RET(apply_A64(pb, h, qv, part));
+            MGPU_RET(apply_A64(pb, h, qv, dot));
         pb.prof.begin(MGPU_KT_MAP, s);
-        k_coeff<<<nseg, kRB, 0, s>>>(part, wg0, S, state, flag);
-        MGPU_LAUNCHED();
+        // g2pix slots of a fused iteration: read, and written for the next
+        // (blocks of iterations have an even length, so a captured one repeats)
+        const int cur = !fused || launched % 2 ? S_G2PIX : S_G2PIXP, nxt = cur == S_G2PIX ? S_G2PIXP : S_G2PIX;
+        if (!fused) {
+            k_coeff<<<nseg, kRB, 0, s>>>(dot, wg0, S, state, flag);
+            MGPU_LAUNCHED();
+        }
         if (two) {
-            k_update_xg<<<nwg, kMB, 0, s>>>(x, h, g, gp, qv, wseg, wq0, sq, S, state, flag);
+            const auto k = fused ? k_update_xg<true> : k_update_xg<false>;
+            k<<<nwg, kMB, 0, s>>>(x, h, g, gp, qv, wseg, wq0, sq, S, state, flag, dot, wg0, cur);
             MGPU_LAUNCHED();
             MGPU_RET(twolvl_apply(pb, g, gp, Cg, nullptr, part, false, state, flag));
         } else {
-            k_update<<<nwg, kMB, 0, s>>>(x, h, g, gp, qv, pb.pc.d_inv, Cg, wseg, wq0, sq, S, state, part, flag);
+            const auto k = fused ? k_update<true> : k_update<false>;
+            k<<<nwg, kMB, 0, s>>>(x, h, g, gp, qv, pb.pc.d_inv, Cg, wseg, wq0, sq, S, state, part, flag, dot, wg0,
+                                  cur);
             MGPU_LAUNCHED();
         }
         pb.prof.end(s);
@@ -790,9 +863,14 @@ int pcg_run(Problem &pb, const double *d_signal, const double *d_noise, double t
             pb.prof.end(s);
         }
         pb.prof.begin(MGPU_KT_MAP, s);
-        k_scalars<<<nseg, kRB, 0, s>>>(part, nwg, wg0, S, d_hist, maxiter, state, nseg, flag, kind, adaptive ? 1 : 0);
-        MGPU_LAUNCHED();
-        k_hupdate<<<nwg, kMB, 0, s>>>(h, Cg, wseg, wq0, sq, S, state, flag);
+        if (!fused) {
+            k_scalars<<<nseg, kRB, 0, s>>>(part, nwg, wg0, S, d_hist, maxiter, state, nseg, flag, kind,
+                                           adaptive ? 1 : 0);
+            MGPU_LAUNCHED();
+        }
+        const auto kh = fused ? k_hupdate<true> : k_hupdate<false>;
+        kh<<<nwg, kMB, 0, s>>>(h, Cg, mixed ? pb.d_mapf : nullptr, wseg, wq0, sq, S, state, flag, part, nwg, wg0, cur,
+                               nxt, d_hist, maxiter, nseg, kind, adaptive ? 1 : 0);
         MGPU_LAUNCHED();
         pb.prof.end(s);
         return MGPU_OK;

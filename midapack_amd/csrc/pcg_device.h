@@ -17,7 +17,7 @@ enum {
     S_GAMMA,
     S_COEFF,
     S_POLAK,
-    S_G2PIXP,
+    S_G2PIXP,   // g2pix of the iteration before (fused sums: the two slots alternate)
     S_K,        // iteration counter (as double)
     S_TOL,
     S_STOPK,    // stop_after (0 = off)
@@ -85,6 +85,48 @@ __device__ __forceinline__ double reduce_parts(const double *__restrict__ p, int
     double t = 0.0;
     for (int w = 0; w < kRB / 64; w++) t += red[w];
     return t;
+}
+
+// Largest number of partials of a segment that the map kernels sum themselves
+// (fused_sums): every workgroup then reads them all, four loads a thread and
+// set, which costs about 1 us against 4.3-7.3 us and a launch for a reduction
+// kernel.  A segment of 1024 workgroups is a map of 262144 pixels; with the
+// 4096 of a 1024^2 map the reads (32 KB a set and workgroup) would add more
+// than the kernel's own traffic.
+constexpr int kFusedParts = 1024;
+
+// reduce_parts for NS sets of nparts <= kFusedParts partials (set k at p + k
+// stride) by a workgroup of kMB threads, in reduce_parts' order and so with its
+// bits: thread t holds the values of its threads t, t + kMB, ...  red: NS * kRB
+// / 64 doubles of LDS; every thread gets the sums.
+template <int NS>
+__device__ __forceinline__ void reduce_parts_wg(const double *__restrict__ p, int64_t stride, int nparts, double *red,
+                                                double (&out)[NS]) {
+    constexpr int J = kRB / kMB, W = kRB / 64;
+    double v[NS][J];
+#pragma unroll
+    for (int k = 0; k < NS; k++)
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const int i = (int) threadIdx.x + j * kMB;
+            v[k][j] = i < nparts ? p[k * stride + i] : 0.0;
+        }
+#pragma unroll
+    for (int k = 0; k < NS; k++)
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            double s = 0.0 + v[k][j];
+            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+            if ((threadIdx.x & 63) == 0) red[k * W + (threadIdx.x >> 6) + j * (kMB / 64)] = s;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+        double t = 0.0;
+#pragma unroll
+        for (int w = 0; w < W; w++) t += red[k * W + w];
+        out[k] = t;
+    }
 }
 
 // pixel handled by this thread of a map-domain workgroup, its segment and the segment end
