@@ -93,10 +93,9 @@ int solve_items(mgpu_batch_item *items, const std::vector<int> &idx, const std::
         lam_max = std::max(lam_max, it.lambda);
         maxit = std::max(maxit, maxiter[r]);
         tol_max = std::max(tol_max, tol[r]);
-        int64_t nmax = 0;
-        for (int b = 0; b < it.nb; b++) nmax = std::max<int64_t>(nmax, it.local_blocks_sizes[b]);
         // the tile length the item would use alone (its own block-length profile)
-        l2[r] = toeplitz_tile_log2(it.lambda, nmax, gopt.tile_log2);
+        l2[r] = toeplitz_tile_log2(it.lambda, it.local_blocks_sizes, it.nb, gopt.precision == MGPU_MIXED,
+                                   gopt.tile_log2);
     }
     const int64_t M = off[R];
     MGPU_ARG(M < (int64_t) INT32_MAX, "batch of %lld padded samples exceeds 2^31-1: split it", (long long) M);
@@ -267,9 +266,10 @@ int pcg_batch_impl(mgpu_batch_item *items, const std::vector<int> &all, const st
     std::map<int, std::vector<int>> groups;  // key: 0 = tiled, 1 = diagonal, lambda + 1 = direct
     for (int k = 0; k < (int) all.size(); k++) {
         const mgpu_batch_item &it = items[all[k]];
-        int64_t nmax = 0;
-        for (int b = 0; b < it.nb; b++) nmax = std::max<int64_t>(nmax, it.local_blocks_sizes[b]);
-        const int l2 = it.lambda > 1 ? toeplitz_tile_log2(it.lambda, nmax, opt ? opt->tile_log2 : 0) : 0;
+        const int l2 = it.lambda > 1 ? toeplitz_tile_log2(it.lambda, it.local_blocks_sizes, it.nb,
+                                                          opt && opt->precision == MGPU_MIXED,
+                                                          opt ? opt->tile_log2 : 0)
+                                     : 0;
         const int key = it.lambda == 1 ? 1 : (l2 > 0 ? 0 : it.lambda + 1);
         groups[key].push_back(k);
     }

@@ -610,7 +610,7 @@ int noalloc_scratch_init(int device);
 int toeplitz_apply_noalloc(Problem &pb, const double *d_in, double *d_out, hipStream_t stream);
 int tile_variant_count(bool fp32, int log2n);
 // real tile length 2^k the plan of a lambda / longest block would use (0: no tiles)
-int toeplitz_tile_log2(int lambda, int64_t nmax, int forced);
+int toeplitz_tile_log2(int lambda, const int *block_sizes, int nb, bool fp32, int forced);
 const char *tile_variant_desc(bool fp32, int log2n, int variant);
 
 int precond_build(Problem &pb, double *d_signal);

@@ -524,10 +524,11 @@ __global__ __launch_bounds__((1 << LOGNC) >> LOGV, MINW) void k_tiles(TileArgs a
             spectral_pair<R>(re[r], im[r], re[RL + RL - 1 - r], im[RL + RL - 1 - r], cf[k], cf[NC - k]);
         }
     } else if (t != 0) {
-        // the coefficients are loaded SG pairs at a time, the next group's loads
+        // the coefficients are loaded SG pairs at a time (2 with 16 values per lane:
+        // 134-148 VGPRs instead of 160-168), the next group's loads
         // issued before the current group's arithmetic (with a scheduling fence
         // after every pair their L2 latencies would add up one after the other)
-        constexpr int SG = RL < MGPU_SPEC_GROUP ? RL : MGPU_SPEC_GROUP;
+        constexpr int SG = LOGV == 4 ? 2 : RL < MGPU_SPEC_GROUP ? RL : MGPU_SPEC_GROUP;
         static_assert(RL % SG == 0, "coefficient groups must tile the paired slots");
         Cx<R> cp[2][SG], cq[2][SG];
 #pragma unroll
@@ -1167,18 +1168,59 @@ static int max_log2n(bool fp32) { return fp32 ? 16 : 15; }
 static std::vector<TileDesc> xcd_order(const std::vector<TileDesc> &t) { return deal_to_xcds(t); }
 static int min_log2n() { return 10; }
 
-// tile length choice: minimise N (log2 N + c) / L over the sizes that fit LDS
-static int choose_log2n(int lambda, int64_t nmax, bool fp32, int forced);
-
-int toeplitz_tile_log2(int lambda, int64_t nmax, int forced) {
-    return lambda > 1 ? choose_log2n(lambda, nmax, false, forced) : 0;
+// Time of a launch of `tiles` tiles of 2^log2n samples with the default variants:
+// that of a few tiles (latency) plus a rate, fitted (us) to 12 ... 18688 tiles on
+// 0.26 M ... 17 M samples in bands of 64, 1024 and 4096, within 15 % of most.
+// FP64 tiles of 32768 samples fill a CU each, so their launches take whole
+// rounds of 256.
+static double tile_launch_us(bool fp32, int log2n, int64_t tiles) {
+    struct Cost {
+        double few, each;
+    };
+    static const Cost c64[] = {{6.4, 0.0028}, {8.7, 0.0050}, {9.3, 0.0093}, {12.8, 0.0225}, {19.5, 0.0455}};
+    static const Cost c32[] = {{6.2, 0.0016}, {9.2, 0.0028}, {9.8, 0.0048}, {12.3, 0.0128}, {16.5, 0.0235}, {22.3, 0.0585}};
+    if (!fp32 && log2n == 15) return 3.0 + 33.0 * (double) ((tiles + 255) / 256);
+    const Cost &c = (fp32 ? c32 : c64)[log2n - 10];
+    return c.few + c.each * (double) tiles;
 }
 
-static int choose_log2n(int lambda, int64_t nmax, bool fp32, int forced) {
+// Tile length for the blocks of one band: the least launch time over the lengths
+// that hold it, by the problem's own block lengths (a batch item has the length
+// of its solo solve).  Short tiles spread a small problem over the chip (12
+// tiles of 32768 samples take 29 us where 128 of 4096 take 9 us: 4 x 65536
+// samples, band 1024) and let several workgroups share a CU, so that one's
+// memory phases overlap another's arithmetic (16 x 2^20 samples, band 1024,
+// FP64: 32768 samples 107 us, 16384 76 us, 8192 73 us, 4096 84 us); long tiles
+// lose less to the overlap of 2(lambda-1) samples (band 4096 on the same
+// samples: 110 us against 111 us).  `forced`: the caller's length.
+static int choose_log2n(int lambda, const std::vector<int> &blocks, bool fp32, int forced) {
+    if (forced > 0) return forced;
+    int best = -1;
+    double best_us = 1e300;
+    for (int l2 = min_log2n(); l2 <= max_log2n(false); l2++) {
+        const int64_t L = ((int64_t) 1 << l2) - 2 * ((int64_t) lambda - 1);
+        if (L < 1) continue;
+        int64_t tiles = 0;
+        for (int n : blocks) tiles += (n + L - 1) / L;
+        const double us = tile_launch_us(fp32, l2, tiles);
+        if (us < best_us) {
+            best_us = us;
+            best = l2;
+        }
+    }
+    return best;
+}
+
+int toeplitz_tile_log2(int lambda, const int *block_sizes, int nb, bool fp32, int forced) {
+    return lambda > 1 ? choose_log2n(lambda, std::vector<int>(block_sizes, block_sizes + nb), fp32, forced) : 0;
+}
+
+// FP32 length that the autotuner may use instead: fewest FFT operations per useful sample
+static int choose_long_log2n(int lambda, int64_t nmax, int forced) {
     if (forced > 0) return forced;
     int best = -1;
     double best_cost = 1e300;
-    for (int l2 = min_log2n(); l2 <= max_log2n(fp32); l2++) {
+    for (int l2 = min_log2n(); l2 <= max_log2n(true); l2++) {
         const double N = (double) (1 << l2);
         const double L = N - 2.0 * (lambda - 1);
         if (L < 1) continue;
@@ -1363,13 +1405,17 @@ int toeplitz_plan(Problem &pb, const int *block_sizes, int nb, int lambda, const
         MGPU_HIP(hipStreamSynchronize(s));
     }
     // tile length of every block: the caller's, or the choice for its band and
-    // the longest block of that band; blocks without a tile length take the direct product
-    std::map<int, int64_t> nmax_of;
-    for (int b = 0; b < nb; b++) nmax_of[lam[b]] = std::max<int64_t>(nmax_of[lam[b]], block_sizes[b]);
+    // the blocks of that band; blocks without a tile length take the direct product
+    std::map<int, int> l2_of;
+    if (!block_log2n) {
+        std::map<int, std::vector<int>> blocks_of;
+        for (int b = 0; b < nb; b++) blocks_of[lam[b]].push_back(block_sizes[b]);
+        for (auto &kv : blocks_of)
+            l2_of[kv.first] = choose_log2n(kv.first, kv.second, fp32, std::min(pb.opt.tile_log2, max_log2n(false)));
+    }
     std::vector<int> l2b((size_t) nb, -1);
     for (int b = 0; b < nb; b++) {
-        int l2 = block_log2n ? block_log2n[b]
-                             : choose_log2n(lam[b], nmax_of[lam[b]], false, std::min(pb.opt.tile_log2, max_log2n(false)));
+        int l2 = block_log2n ? block_log2n[b] : l2_of[lam[b]];
         if (l2 < min_log2n() || l2 > max_log2n(false) || (1 << l2) - 2 * (lam[b] - 1) < 1) l2 = -1;
         l2b[b] = l2;
     }
@@ -1442,9 +1488,11 @@ int toeplitz_plan(Problem &pb, const int *block_sizes, int nb, int lambda, const
                                                                                  C.d_coefW32);
             MGPU_LAUNCHED();
         }
-        // FP32 products of a mixed solve: a longer tile when it costs fewer FFT
-        // operations per useful sample (FP32 halves the registers and LDS a tile needs)
-        const int l2f = fp32 ? choose_log2n(C.lambda, nmax_c, true, pb.opt.tile_log2) : -1;
+        // FP32 products of a mixed solve under the autotuner: a longer tile when it costs
+        // fewer FFT operations per useful sample (FP32 halves the registers and LDS a tile needs)
+        const int l2f = fp32 && pb.opt.tile_variant == MGPU_TILE_AUTOTUNE
+                                ? choose_long_log2n(C.lambda, nmax_c, pb.opt.tile_log2)
+                                : -1;
         if (l2f > C.log2n && l2f <= max_log2n(true)) {
             const int Nf = 1 << l2f, NCf = Nf / 2;
             C.log2n32 = l2f;
@@ -1505,7 +1553,8 @@ struct TileShape {
 };
 
 static const TileShape kShapes64_9[] = {{3, 3, true, 1, false}};
-static const TileShape kShapes64_mid[] = {{4, 4, true, 1, false}, {3, 3, true, 1, false}};
+static const TileShape kShapes64_mid[] = {{4, 4, true, 1, false}, {3, 3, true, 1, false}, {4, 4, false, 1, false}};
+static const TileShape kShapes64_13[] = {{4, 4, true, 1, false}, {3, 3, true, 1, false}, {5, 5, false, 2, false}};
 static const TileShape kShapes64_14[] = {{5, 4, false, 1, false}, {5, 5, false, 1, false}, {4, 4, false, 1, false},
                                          {5, 5, false, 1, true}};
 static const TileShape kShapes32_14[] = {{5, 4, true, 1, false}, {5, 5, true, 1, false}, {4, 4, true, 1, false},
@@ -1520,7 +1569,8 @@ static const TileShape *tile_shapes(bool fp32, int log2n, int *n) {
         return a;                               \
     } while (0)
     if (lognc == 9) MGPU_SHAPES(kShapes64_9);
-    if (lognc >= 10 && lognc <= 13) MGPU_SHAPES(kShapes64_mid);
+    if (lognc >= 10 && lognc <= 12) MGPU_SHAPES(kShapes64_mid);
+    if (lognc == 13) MGPU_SHAPES(kShapes64_13);
     if (lognc == 14) {
         if (fp32) MGPU_SHAPES(kShapes32_14);
         MGPU_SHAPES(kShapes64_14);
@@ -1626,15 +1676,19 @@ static int launch_tiles(Problem &pb, const TileClass &C, const R *d_in, R *d_out
         case 9: MGPU_TL(9, 3, 3, true, 1);
         case 10:
             if (variant == 2) MGPU_TL(10, 3, 3, true, 1);
+            if (variant == 3) MGPU_TL(10, 4, 4, false, 1);
             MGPU_TL(10, 4, 4, true, 1);
         case 11:
             if (variant == 2) MGPU_TL(11, 3, 3, true, 1);
+            if (variant == 3) MGPU_TL(11, 4, 4, false, 1);
             MGPU_TL(11, 4, 4, true, 1);
         case 12:
             if (variant == 2) MGPU_TL(12, 3, 3, true, 1);
+            if (variant == 3) MGPU_TL(12, 4, 4, false, 1);
             MGPU_TL(12, 4, 4, true, 1);
         case 13:
             if (variant == 2) MGPU_TL(13, 3, 3, true, 1);
+            if (variant == 3) MGPU_TL(13, 5, 5, false, 2);
             MGPU_TL(13, 4, 4, true, 1);
         case 14:
             if constexpr (F32) {
@@ -1665,9 +1719,14 @@ static int launch_tiles(Problem &pb, const TileClass &C, const R *d_in, R *d_out
 // unless the caller forces another or opts into autotuning.  FP64 results
 // therefore depend only on the inputs (variants differ in pass structure and
 // round differently).  The entries are the fastest variants measured on
-// MI355X for the lengths the workloads use (the variant tables above).
+// MI355X with the chip filled: at 2048 to 8192 samples the one-plane exchange,
+// whose half LDS lets registers alone limit a CU to three waves a SIMD (8192
+// samples, 2736 tiles: 88.6 -> 73.3 us FP64, 47.9 -> 46.0 us FP32); at 16384
+// samples 32 values a lane, so that four waves hold a tile and two or more
+// tiles share a CU (2048 tiles: 148 -> 111 us FP64, 77 -> 62 us FP32).
 static int default_variant(bool fp32, int log2n) {
     const int lognc = log2n - 1;
+    if (lognc >= 10 && lognc <= 13) return 3;
     if (!fp32 && lognc == 14) return 2;
     if (fp32 && lognc == 14) return 5;
     return 1;
