@@ -16,12 +16,18 @@
 // a bounded Levenberg-Marquardt runs one workgroup per block on the device.
 // Both minimise the same objective; results agree to the fit tolerance.
 //
-// FFTs: batched radix-2 Stockham passes in HBM (one launch per pass) for
-// power-of-two n; other n use Bluestein's chirp-z transform on the next
-// power of two >= 2n - 1.  The forward transform of the periodogram and the
-// inverse transform of psdm1 (real and even, so its inverse DFT is its
-// forward DFT divided by n) share the same machinery.  This is set-up work
-// (once per noise model), not the PCG hot path.
+// FFTs: batched Stockham passes in HBM, four radix-2 stages a launch in
+// registers (k_fft_step), for power-of-two n; other n use Bluestein's chirp-z
+// transform on the next power of two >= 2n - 1.  The forward transform of the
+// periodogram and the inverse transform of psdm1 (real and even, so its
+// inverse DFT is its forward DFT divided by n) share the same machinery.
+//
+// Sums over a block's samples or frequencies (the line fit of the detrending,
+// the window's power, the normal equations of the fit) are 256 chains, chain c
+// adding the terms c, c + 256, ... in order, then a fixed tree over the chains.
+// chain_sums computes the terms of 16 chains by 1024 threads and adds them up in
+// that order from LDS, so one block's sum runs on 16 CUs at once with the bits
+// of one workgroup of 256 threads.
 #include "mgpu_internal.h"
 
 #include <algorithm>
@@ -33,24 +39,57 @@ namespace mgpu {
 
 namespace {
 
-// one radix-2 Stockham pass over `batch` transforms of length M = 2^logm:
-// sub-transform size ns -> 2 ns; sign -1 forward, +1 inverse (no scaling)
-__global__ void k_fft_pass(const double2 *__restrict__ in, double2 *__restrict__ out, int logm, int ns, int sign,
-                           int batch) {
-    const int64_t M = (int64_t) 1 << logm, half = M >> 1;
+// LR radix-2 Stockham passes over `batch` transforms of length M = 2^logm in one
+// launch: sub-transform size ns -> ns 2^LR; sign -1 forward, +1 inverse (no
+// scaling).  A thread holds the 2^LR points x[j + t M / 2^LR]; the passes' pairs
+// and twiddles are those of one pass at a time.  REAL: the input is the real
+// sequence xr + xoff[b].  Bound by HBM and the sincospi of the twiddles (15 for
+// 16 points): 64 transforms of 2^17 points, 17 passes of 38 us -> 5 launches of
+// 37-76 us.
+template <int LR, bool REAL>
+__global__ __launch_bounds__(256) void k_fft_step(const double2 *__restrict__ in, const double *__restrict__ xr,
+                                                  const int64_t *__restrict__ xoff, double2 *__restrict__ out,
+                                                  int logm, int ns, int sign, int batch) {
+    constexpr int R = 1 << LR;
+    const int64_t M = (int64_t) 1 << logm, per = M >> LR;
     const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= half * batch) return;
-    const int64_t b = gid / half, j = gid % half;
-    const double2 *x = in + b * M;
-    double2 *y = out + b * M;
-    const int64_t r = j % ns;
-    double s, c;
-    sincospi((double) sign * (double) r / (double) ns, &s, &c);
-    const double2 v0 = x[j], u = x[j + half];
-    const double2 v1 = make_double2(u.x * c - u.y * s, u.x * s + u.y * c);
-    const int64_t d = (j / ns) * ns * 2 + r;
-    y[d] = make_double2(v0.x + v1.x, v0.y + v1.y);
-    y[d + ns] = make_double2(v0.x - v1.x, v0.y - v1.y);
+    if (gid >= per * batch) return;
+    const int64_t b = gid / per, j = gid % per;
+    double2 v[R];
+    if constexpr (REAL) {
+        const double *x = xr + xoff[b];
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t] = make_double2(x[j + t * per], 0.0);
+    } else {
+        const double2 *x = in + b * M;
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t] = x[j + t * per];
+    }
+    const int64_t r = j & (ns - 1);
+    // before stage s, v[t (1 << s) + u] is the point of offset u ns inside a
+    // group of ns 2^s points, t the group's place among the 2^(LR-s) it holds
+#pragma unroll
+    for (int st = 0; st < LR; st++) {
+        double2 o[R];
+        const double nsd = (double) ((int64_t) ns << st);
+#pragma unroll
+        for (int u = 0; u < (1 << st); u++) {
+            double s, c;
+            sincospi((double) sign * (double) (r + (int64_t) u * ns) / nsd, &s, &c);
+#pragma unroll
+            for (int t = 0; t < (R >> (st + 1)); t++) {
+                const double2 v0 = v[(t << st) + u], w = v[((t + (R >> (st + 1))) << st) + u];
+                const double2 v1 = make_double2(w.x * c - w.y * s, w.x * s + w.y * c);
+                o[(t << (st + 1)) + u] = make_double2(v0.x + v1.x, v0.y + v1.y);
+                o[(t << (st + 1)) + u + (1 << st)] = make_double2(v0.x - v1.x, v0.y - v1.y);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t] = o[t];
+    }
+    double2 *y = out + b * M + (j - r) * R + r;
+#pragma unroll
+    for (int t = 0; t < R; t++) y[(int64_t) t * ns] = v[t];
 }
 
 // exp(sign * pi * i * j^2 / n), with j^2 reduced mod 2n exactly
@@ -75,6 +114,7 @@ __global__ void k_blue_prep(const double *__restrict__ x, const int64_t *__restr
     const int64_t b = gid / M, t = gid % M;
     const int64_t n = nlen[b];
     A[gid] = t < n ? cmul(make_double2(x[xoff[b] + t], 0.0), chirp(t, n, -1)) : make_double2(0.0, 0.0);
+    if (!B) return;  // the chirp's spectrum is there already
     double2 v = make_double2(0.0, 0.0);
     if (t < n)
         v = chirp(t, n, +1);
@@ -101,127 +141,208 @@ __global__ void k_blue_post(const double2 *__restrict__ C, const int *__restrict
     X[b * nout_max + k] = make_double2(v.x / (double) M, v.y / (double) M);
 }
 
-// power of two: load the real input as complex
-__global__ void k_real_to_c(const double *__restrict__ x, const int64_t *__restrict__ xoff, int logm, int batch,
-                            double2 *__restrict__ A) {
-    const int64_t M = (int64_t) 1 << logm;
-    const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= M * batch) return;
-    const int64_t b = gid / M, t = gid % M;
-    A[gid] = make_double2(x[xoff[b] + t], 0.0);
-}
+// forward DFTs of `batch` real sequences of lengths nlen[b] (all with the same
+// transform size M = 2^logm: n = M for powers of two, else the Bluestein size),
+// with the work buffers of one group of blocks
+struct Dft {
+    Problem &pb;
+    int logm, batch;
+    bool pow2;
+    int64_t nout_max;
+    double2 *a = nullptr, *b = nullptr, *c = nullptr;  // c: the chirp's spectrum (Bluestein), kept between transforms
+    double2 *X = nullptr;                              // [batch * stride] the transform
+    int64_t stride = 0;
+    bool have_chirp = false;
 
-struct Buf {
-    Arena &ar;
-    double2 *p = nullptr;
-    explicit Buf(Arena &a) : ar(a) {}
-    ~Buf() {
-        if (p) ar.release(p);
+    Dft(Problem &p, int logm_, int batch_, bool pow2_, int64_t nout)
+        : pb(p), logm(logm_), batch(batch_), pow2(pow2_), nout_max(nout) {}
+    ~Dft() {
+        for (double2 *p : {a, b, c})
+            if (p) pb.arena.release(p);
+    }
+    int alloc() {
+        const size_t total = ((size_t) 1 << logm) * batch;
+        MGPU_RET(pb.arena.alloc(&a, total));
+        MGPU_RET(pb.arena.alloc(&b, total));
+        if (!pow2) MGPU_RET(pb.arena.alloc(&c, total));
+        return MGPU_OK;
+    }
+    // transform of src (or of the real sequences xr + xoff[b]) through tmp: src holds the result
+    int fft(double2 *&src, double2 *&tmp, int sign, const double *xr, const int64_t *xoff) {
+        const int64_t M = (int64_t) 1 << logm;
+        for (int done = 0; done < logm;) {
+            const int lr = std::min(4, logm - done), ns = 1 << done;
+            const unsigned g = grid_for((M >> lr) * batch, 256);
+            hipStream_t s = pb.stream;
+#define MGPU_FFT(LR)                                                                                    \
+    case LR:                                                                                            \
+        if (xr && done == 0)                                                                            \
+            k_fft_step<LR, true><<<g, 256, 0, s>>>(src, xr, xoff, tmp, logm, ns, sign, batch);          \
+        else                                                                                            \
+            k_fft_step<LR, false><<<g, 256, 0, s>>>(src, nullptr, nullptr, tmp, logm, ns, sign, batch); \
+        break
+            switch (lr) {
+                MGPU_FFT(1);
+                MGPU_FFT(2);
+                MGPU_FFT(3);
+                MGPU_FFT(4);
+            }
+#undef MGPU_FFT
+            MGPU_LAUNCHED();
+            std::swap(src, tmp);
+            done += lr;
+        }
+        return MGPU_OK;
+    }
+    // X[b * stride + k] = DFT_k for k < min(n, nout_max)
+    int run(const double *d_x, const int64_t *d_xoff, const int *d_nlen, double2 *d_out) {
+        hipStream_t s = pb.stream;
+        const int64_t M = (int64_t) 1 << logm, total = M * batch;
+        if (pow2) {
+            MGPU_RET(fft(a, b, -1, d_x, d_xoff));
+            X = a;
+            stride = M;
+            return MGPU_OK;
+        }
+        k_blue_prep<<<grid_for(total, 256), 256, 0, s>>>(d_x, d_xoff, d_nlen, logm, batch, a, have_chirp ? nullptr : c);
+        MGPU_LAUNCHED();
+        MGPU_RET(fft(a, b, -1, nullptr, nullptr));
+        if (!have_chirp) MGPU_RET(fft(c, b, -1, nullptr, nullptr));
+        have_chirp = true;
+        k_pointwise<<<grid_for(total, 256), 256, 0, s>>>(a, c, total);
+        MGPU_LAUNCHED();
+        MGPU_RET(fft(a, b, +1, nullptr, nullptr));
+        k_blue_post<<<grid_for(nout_max * batch, 256), 256, 0, s>>>(a, d_nlen, logm, batch, nout_max, d_out);
+        MGPU_LAUNCHED();
+        X = d_out;
+        stride = nout_max;
+        return MGPU_OK;
     }
 };
 
-// forward DFT of `batch` real sequences of lengths nlen[b] (all with the same
-// transform size M = 2^logm: n = M for powers of two, else the Bluestein
-// size) read at x + xoff[b]; X[b * nout_max + k] = DFT_k for k < n.
-int dft_real(Problem &pb, const double *d_x, const int64_t *d_xoff, const int *d_nlen, int batch, int logm,
-             bool pow2, int64_t nout_max, double2 *d_X) {
-    hipStream_t s = pb.stream;
-    const int64_t M = (int64_t) 1 << logm, total = M * batch;
-    Buf a(pb.arena), b(pb.arena), c(pb.arena);
-    MGPU_RET(pb.arena.alloc(&a.p, (size_t) total));
-    MGPU_RET(pb.arena.alloc(&b.p, (size_t) total));
-    auto fft = [&](double2 *&src, double2 *&tmp, int sign) -> int {
-        for (int ns = 1; ns < M; ns <<= 1) {
-            k_fft_pass<<<grid_for(total / 2, 256), 256, 0, s>>>(src, tmp, logm, ns, sign, batch);
-            MGPU_LAUNCHED();
-            std::swap(src, tmp);
+constexpr int kChains = 256;                       // chains of a sum
+constexpr int kChainCols = 16;                     // chains of a workgroup
+constexpr int kChainRows = 64;                     // terms of a chain computed at once
+constexpr int kChainWG = kChainCols * kChainRows;  // threads
+constexpr int kChainGroups = kChains / kChainCols;
+
+// sums over terms 0 .. count-1: chain c of `group` (c = 16 group + lane) adds its
+// terms c, c + 256, ... in order.  term(i, v) gives the NV values of term i, and
+// sum s of the NS adds v[ia(s)] * v[ib(s)] (ib < 0: v[ia(s)] itself).  out[s *
+// kChains + c].  The terms of 64 rows go to LDS, are added by the first NS * 16
+// threads while all compute the next 64 (two buffers, one barrier a turn).
+template <int NV, int NS, typename Term, typename Pair>
+__device__ __forceinline__ void chain_sums(int64_t count, int group, Term term, Pair pair, double *__restrict__ out) {
+    static_assert(NS * kChainCols <= kChainWG, "one thread per chain and sum");
+    __shared__ double buf[2][kChainRows][NV][kChainCols];
+    const int t = threadIdx.x, col = t % kChainCols, row = t / kChainCols;
+    const int s = t / kChainCols;  // sum of a summing thread (its chain is col)
+    int ia = 0, ib = -1;
+    if (s < NS) pair(s, ia, ib);
+    double acc = 0.0;
+    const int64_t c = (int64_t) group * kChainCols + col;
+    const int64_t rows = (count + kChains - 1) / kChains;
+    for (int64_t r0 = 0, turn = 0; r0 < rows; r0 += kChainRows, turn++) {
+        double(*bf)[NV][kChainCols] = buf[turn & 1];
+        const int64_t i = (r0 + row) * kChains + c;
+        if (i < count) {
+            double v[NV];
+            term(i, v);
+#pragma unroll
+            for (int k = 0; k < NV; k++) bf[row][k][col] = v[k];
         }
-        return MGPU_OK;
-    };
-    if (pow2) {
-        k_real_to_c<<<grid_for(total, 256), 256, 0, s>>>(d_x, d_xoff, logm, batch, a.p);
-        MGPU_LAUNCHED();
-        MGPU_RET(fft(a.p, b.p, -1));
-        // a.p holds the spectrum (pointers swapped in place)
-        MGPU_HIP(hipMemcpy2DAsync(d_X, sizeof(double2) * nout_max, a.p, sizeof(double2) * M,
-                                  sizeof(double2) * std::min<int64_t>(nout_max, M), batch, hipMemcpyDeviceToDevice, s));
-        MGPU_HIP(hipStreamSynchronize(s));  // before the work buffers go back to the block cache
-        return MGPU_OK;
+        __syncthreads();
+        if (s < NS) {
+            const int64_t left = (count - c + kChains - 1) / kChains - r0;  // terms of the chain from row r0 on
+            const int m = (int) (left < kChainRows ? left : kChainRows);
+#pragma unroll 8
+            for (int q = 0; q < m; q++) {
+                const double x = bf[q][ia][col];
+                acc += ib < 0 ? x : x * bf[q][ib][col];
+            }
+        }
     }
-    MGPU_RET(pb.arena.alloc(&c.p, (size_t) total));
-    k_blue_prep<<<grid_for(total, 256), 256, 0, s>>>(d_x, d_xoff, d_nlen, logm, batch, a.p, c.p);
-    MGPU_LAUNCHED();
-    MGPU_RET(fft(a.p, b.p, -1));
-    MGPU_RET(fft(c.p, b.p, -1));
-    k_pointwise<<<grid_for(total, 256), 256, 0, s>>>(a.p, c.p, total);
-    MGPU_LAUNCHED();
-    MGPU_RET(fft(a.p, b.p, +1));
-    k_blue_post<<<grid_for(nout_max * batch, 256), 256, 0, s>>>(a.p, d_nlen, logm, batch, nout_max, d_X);
-    MGPU_LAUNCHED();
-    MGPU_HIP(hipStreamSynchronize(s));  // before the work buffers go back to the block cache
-    return MGPU_OK;
+    if (s < NS) out[s * kChains + c] = acc;
+}
+
+// the tree over 256 chains that a workgroup of 256 threads would run (halves
+// added pairwise), by one wave: every lane gets the sum
+__device__ __forceinline__ double chain_tree(const double *__restrict__ v) {
+    const int l = threadIdx.x & 63;
+    double a = (v[l] + v[l + 128]) + (v[l + 64] + v[l + 192]);
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o);
+    return __shfl(a, 0);
+}
+
+// sums of x and t x over a block (the least-squares line): parts[b][2][256]
+__global__ __launch_bounds__(kChainWG) void k_line_sums(const double *__restrict__ noise,
+                                                        const int64_t *__restrict__ start,
+                                                        const int *__restrict__ nlen, const int *__restrict__ blocks,
+                                                        double *__restrict__ parts) {
+    const int bi = blockIdx.x / kChainGroups, g = blockIdx.x % kChainGroups;
+    const double *x = noise + start[blocks[bi]];
+    chain_sums<2, 2>(
+            nlen[bi], g,
+            [&](int64_t t, double *v) {
+                v[0] = x[t];
+                v[1] = (double) t * x[t];
+            },
+            [](int s, int &ia, int &ib) { ia = s; }, parts + (int64_t) bi * 2 * kChains);
 }
 
 // detrended, Hann-windowed segment: xw[t] = w_t (x_t - (c0 + c1 t)), the line
-// fitted by least squares (scipy.signal.detrend type 'linear'); one workgroup per block
-__global__ __launch_bounds__(256) void k_detrend_window(const double *__restrict__ noise,
-                                                        const int64_t *__restrict__ start,
-                                                        const int *__restrict__ nlen, const int *__restrict__ blocks,
-                                                        const int64_t *__restrict__ xoff, double *__restrict__ xw,
-                                                        double *__restrict__ wsum2) {
-    __shared__ double red[256];
-    const int bi = blockIdx.x;
+// fitted by least squares (scipy.signal.detrend type 'linear'), and the chains of
+// sum w^2: wparts[b][256]
+__global__ __launch_bounds__(kChainWG) void k_detrend_window(const double *__restrict__ noise,
+                                                             const int64_t *__restrict__ start,
+                                                             const int *__restrict__ nlen,
+                                                             const int *__restrict__ blocks,
+                                                             const int64_t *__restrict__ xoff,
+                                                             const double *__restrict__ parts,
+                                                             double *__restrict__ xw, double *__restrict__ wparts) {
+    const int bi = blockIdx.x / kChainGroups, g = blockIdx.x % kChainGroups;
     const int64_t n = nlen[bi];
     const double *x = noise + start[blocks[bi]];
-    // sums for the line fit over t = 0..n-1
-    double sx = 0.0, stx = 0.0;
-    for (int64_t t = threadIdx.x; t < n; t += 256) {
-        sx += x[t];
-        stx += (double) t * x[t];
-    }
-    auto tree = [&](double v) {
-        red[threadIdx.x] = v;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if ((int) threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
-        }
-        const double r = red[0];
-        __syncthreads();
-        return r;
-    };
-    sx = tree(sx);
-    stx = tree(stx);
+    double *__restrict__ o = xw + xoff[bi];
+    const double sx = chain_tree(parts + (int64_t) bi * 2 * kChains);
+    const double stx = chain_tree(parts + ((int64_t) bi * 2 + 1) * kChains);
     const double dn = (double) n;
     const double st = dn * (dn - 1.0) / 2.0, stt = (dn - 1.0) * dn * (2.0 * dn - 1.0) / 6.0;
     const double det = dn * stt - st * st;
     const double c1 = (dn * stx - st * sx) / det, c0 = (sx - c1 * st) / dn;
-    double w2 = 0.0;
-    for (int64_t t = threadIdx.x; t < n; t += 256) {
-        double sn, cs;
-        sincospi(2.0 * (double) t / dn, &sn, &cs);
-        const double w = 0.5 - 0.5 * cs;  // periodic Hann
-        xw[xoff[bi] + t] = w * (x[t] - (c0 + c1 * (double) t));
-        w2 += w * w;
-    }
-    w2 = tree(w2);
-    if (threadIdx.x == 0) wsum2[bi] = w2;
+    chain_sums<1, 1>(
+            n, g,
+            [&](int64_t t, double *v) {
+                double sn, cs;
+                sincospi(2.0 * (double) t / dn, &sn, &cs);
+                const double w = 0.5 - 0.5 * cs;  // periodic Hann
+                o[t] = w * (x[t] - (c0 + c1 * (double) t));
+                v[0] = w * w;
+            },
+            [](int, int &ia, int &) { ia = 0; }, wparts + (int64_t) bi * kChains);
+}
+
+__global__ __launch_bounds__(64) void k_chain_tree(const double *__restrict__ parts, double *__restrict__ out) {
+    const double v = chain_tree(parts + (int64_t) blockIdx.x * kChains);
+    if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
 // log10 of the one-sided density periodogram, k = 1 .. n/2
-__global__ void k_logpsd(const double2 *__restrict__ X, const int *__restrict__ nlen, int64_t nout_max, int batch,
-                         const double *__restrict__ wsum2, double fsamp, double *__restrict__ y) {
+// (y of block blocks[b] at yoff[blocks[b]])
+__global__ void k_logpsd(const double2 *__restrict__ X, int64_t stride, const int *__restrict__ nlen, int64_t nmax,
+                         int batch, const double *__restrict__ wsum2, double fsamp, const int *__restrict__ blocks,
+                         const int64_t *__restrict__ yoff, double *__restrict__ y) {
     const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t half = nout_max / 2 + 1;
+    const int64_t half = nmax / 2 + 1;
     if (gid >= half * batch) return;
     const int64_t b = gid / half, k = gid % half;
     const int64_t n = nlen[b];
     if (k > n / 2) return;
-    const double2 v = X[b * nout_max + k];
+    const double2 v = X[b * stride + k];
     double p = (v.x * v.x + v.y * v.y) / (fsamp * wsum2[b]);
     const bool nyq = (n % 2 == 0) && k == n / 2;
     if (k > 0 && !nyq) p *= 2.0;
-    y[b * half + k] = log10(p);
+    y[yoff[blocks[b]] + k] = log10(p);
 }
 
 // model pieces at frequency f: h = log10(1 + g), g = u^alpha, u = (f + fmin) / fknee
@@ -243,158 +364,201 @@ __device__ __forceinline__ Model model_at(double f, double alpha, double fknee, 
 
 constexpr int kFitIter = 400;
 
-// bounded Levenberg-Marquardt fit of a + log10(1 + ((f+fmin)/fknee)^alpha) to y[1..n/2];
-// one workgroup per block; params[4b..4b+3] = (a, alpha, fknee, fmin)
-__global__ __launch_bounds__(256) void k_fit(const double *__restrict__ y, const int *__restrict__ nlen,
-                                             int64_t nout_max, double fsamp, double *__restrict__ params) {
-    __shared__ double red[256];
-    __shared__ double sh[20];
-    const int b = blockIdx.x;
-    const int64_t n = nlen[b], half = nout_max / 2 + 1, K = n / 2;
-    const double *yb = y + b * half;
-    const double lo[4] = {-20.0, -10.0, 1e-12, 0.0}, hi[4] = {0.0, 0.0, 20.0, 1.0};
-    double p[4] = {-7.0, -1.0, 0.1, 1e-6};
-    auto tree = [&](double v) {
-        red[threadIdx.x] = v;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if ((int) threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
-        }
-        const double r = red[0];
-        __syncthreads();
-        return r;
-    };
-    auto cost_at = [&](const double *q) {
-        double c = 0.0;
-        for (int64_t k = 1 + threadIdx.x; k <= K; k += 256) {
-            const double f = (double) k * fsamp / (double) n;
-            const double r = q[0] + model_at(f, q[1], q[2], q[3]).h - yb[k];
-            c += r * r;
-        }
-        return tree(c);
-    };
-    double cost = cost_at(p);
-    double mu = 1e-3;
-    for (int it = 0; it < kFitIter; it++) {
-        // normal equations J^T J (10 entries) and J^T r (4)
-        double acc[14] = {0};
-        for (int64_t k = 1 + threadIdx.x; k <= K; k += 256) {
-            const double f = (double) k * fsamp / (double) n;
-            const Model md = model_at(f, p[1], p[2], p[3]);
-            const double r = p[0] + md.h - yb[k];
-            const double J[4] = {1.0, md.dh_alpha, md.dh_fknee, md.dh_fmin};
-            int e = 0;
-            for (int i = 0; i < 4; i++)
-                for (int j = i; j < 4; j++) acc[e++] += J[i] * J[j];
-            for (int i = 0; i < 4; i++) acc[10 + i] += J[i] * r;
-        }
-        for (int e = 0; e < 14; e++) {
-            const double v = tree(acc[e]);
-            if (threadIdx.x == 0) sh[e] = v;
-        }
-        __syncthreads();
-        // thread 0: damped step (J^T J + mu diag) d = -J^T r, projected on the bounds
-        if (threadIdx.x == 0) {
-            double A[4][4], g[4];
-            int e = 0;
-            for (int i = 0; i < 4; i++)
-                for (int j = i; j < 4; j++) {
-                    A[i][j] = sh[e];
-                    A[j][i] = sh[e];
-                    e++;
-                }
-            for (int i = 0; i < 4; i++) g[i] = -sh[10 + i];
-            for (int i = 0; i < 4; i++) A[i][i] += mu * (A[i][i] > 0.0 ? A[i][i] : 1.0);
-            // active set: a parameter on a bound whose descent direction points
-            // outside stays fixed (its row and column leave the system)
-            for (int i = 0; i < 4; i++) {
-                const bool act = (p[i] <= lo[i] && g[i] < 0.0) || (p[i] >= hi[i] && g[i] > 0.0);
-                if (act) {
-                    for (int j = 0; j < 4; j++) {
-                        A[i][j] = 0.0;
-                        A[j][i] = 0.0;
-                    }
-                    A[i][i] = 1.0;
-                    g[i] = 0.0;
-                }
-            }
-            // Gaussian elimination with partial pivoting (4x4)
-            for (int c = 0; c < 4; c++) {
-                int pr = c;
-                for (int r = c + 1; r < 4; r++)
-                    if (fabs(A[r][c]) > fabs(A[pr][c])) pr = r;
-                for (int j = 0; j < 4; j++) {
-                    const double t = A[c][j];
-                    A[c][j] = A[pr][j];
-                    A[pr][j] = t;
-                }
-                const double tg = g[c];
-                g[c] = g[pr];
-                g[pr] = tg;
-                for (int r = c + 1; r < 4; r++) {
-                    const double fct = A[c][c] != 0.0 ? A[r][c] / A[c][c] : 0.0;
-                    for (int j = c; j < 4; j++) A[r][j] -= fct * A[c][j];
-                    g[r] -= fct * g[c];
-                }
-            }
-            double d[4];
-            for (int r = 3; r >= 0; r--) {
-                double v = g[r];
-                for (int j = r + 1; j < 4; j++) v -= A[r][j] * d[j];
-                d[r] = A[r][r] != 0.0 ? v / A[r][r] : 0.0;
-            }
-            double dn = 0.0, pn = 0.0;
-            for (int i = 0; i < 4; i++) {
-                const double q = fmin(fmax(p[i] + d[i], lo[i]), hi[i]);
-                sh[15 + i] = q;
-                dn += (q - p[i]) * (q - p[i]);
-                pn += p[i] * p[i];
-            }
-            sh[19] = sqrt(dn) <= 1e-14 * (sqrt(pn) + 1e-14) ? 1.0 : 0.0;
-        }
-        __syncthreads();
-        double q[4] = {sh[15], sh[16], sh[17], sh[18]};
-        const bool tiny = sh[19] != 0.0;
-        const double cq = cost_at(q);
-        if (cq < cost) {
-            const double rel = (cost - cq) / fmax(cost, 1e-300);
-            for (int i = 0; i < 4; i++) p[i] = q[i];
-            cost = cq;
-            mu = fmax(mu * 0.3, 1e-12);
-            if (rel < 1e-15 || tiny) break;
-        } else {
-            mu *= 10.0;
-            if (mu > 1e12 || tiny) break;
-        }
-    }
-    if (threadIdx.x == 0)
-        for (int i = 0; i < 4; i++) params[4 * (int64_t) b + i] = p[i];
+// Bounded Levenberg-Marquardt fit of a + log10(1 + ((f+fmin)/fknee)^alpha) to
+// y[1..n/2], every block of the noise model at once.  One evaluation of the
+// model at a block's trial point q gives its cost and, if q is accepted, the
+// normal equations of the next step: k_fit_eval sums both (16 workgroups a
+// block), k_fit_step decides and takes the step.  Bound by the logarithms and
+// exponentials (VALU): on 64 blocks of 2^17 samples one workgroup a block, with
+// two model passes an iteration, took 18.4 ms; 64 evaluations of 28 us and
+// decisions of 6 us take 2.2 ms.
+struct FitState {
+    double p[4], q[4];   // best point, trial point (a, alpha, fknee, fmin)
+    double A[13];        // normal equations at p: J^T J (0..9), J^T r (10..12: its last three)
+    double jr0;          // J^T r, first entry
+    double cost, mu;
+    int it, tiny, done, first;
+};
+
+constexpr int kFitSums = 14;  // 13 products of J and r (below) and the cost
+
+// products of the values (r, dh_alpha, dh_fknee, dh_fmin), J = (1, dh...):
+// J_i J_j for i <= j without 1 * 1, then J_i r, then r r
+__device__ __forceinline__ void fit_pair(int s, int &ia, int &ib) {
+    const int a[kFitSums] = {1, 2, 3, 1, 1, 1, 2, 2, 3, 0, 1, 2, 3, 0};
+    const int b[kFitSums] = {-1, -1, -1, 1, 2, 3, 2, 3, 3, -1, 0, 0, 0, 0};
+    ia = a[s];
+    ib = b[s];
 }
 
-// psdm1 of the fitted model on rfftfreq(n), extended to the full even sequence of length n
-__global__ void k_psdm1_even(const double *__restrict__ params, const int *__restrict__ nlen, int64_t nmax,
-                             int batch, double fsamp, double *__restrict__ out) {
+__global__ void k_fit_init(FitState *__restrict__ st, int nb) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nb) return;
+    FitState &F = st[b];
+    const double p0[4] = {-7.0, -1.0, 0.1, 1e-6};
+    for (int i = 0; i < 4; i++) F.p[i] = F.q[i] = p0[i];
+    F.mu = 1e-3;
+    F.it = F.tiny = F.done = 0;
+    F.first = 1;
+}
+
+__global__ __launch_bounds__(kChainWG) void k_fit_eval(const double *__restrict__ y, const int64_t *__restrict__ yoff,
+                                                       const int *__restrict__ nlen, double fsamp,
+                                                       const FitState *__restrict__ st, double *__restrict__ parts) {
+    const int b = blockIdx.x / kChainGroups, g = blockIdx.x % kChainGroups;
+    if (st[b].done) return;
+    const int64_t n = nlen[b], K = n / 2;
+    const double *yb = y + yoff[b] + 1;
+    const double q0 = st[b].q[0], q1 = st[b].q[1], q2 = st[b].q[2], q3 = st[b].q[3];
+    chain_sums<4, kFitSums>(
+            K, g,
+            [&](int64_t i, double *v) {
+                const double f = (double) (i + 1) * fsamp / (double) n;
+                const Model md = model_at(f, q1, q2, q3);
+                v[0] = q0 + md.h - yb[i];
+                v[1] = md.dh_alpha;
+                v[2] = md.dh_fknee;
+                v[3] = md.dh_fmin;
+            },
+            fit_pair, parts + (int64_t) b * kFitSums * kChains);
+}
+
+// one workgroup per block: sums of the evaluation at q, accept or reject, next
+// trial point; *left counts the blocks that go on
+__global__ __launch_bounds__(64 * kFitSums) void k_fit_step(const double *__restrict__ parts,
+                                                            const int *__restrict__ nlen, FitState *__restrict__ st,
+                                                            int *__restrict__ left) {
+    __shared__ double sh[kFitSums];
+    const int b = blockIdx.x;
+    FitState &F = st[b];
+    if (F.done) return;  // written by this block's thread 0 of an earlier launch only
+    const int wv = threadIdx.x >> 6;
+    const double v = chain_tree(parts + ((int64_t) b * kFitSums + wv) * kChains);
+    if ((threadIdx.x & 63) == 0) sh[wv] = v;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const double lo[4] = {-20.0, -10.0, 1e-12, 0.0}, hi[4] = {0.0, 0.0, 20.0, 1.0};
+    const double cq = sh[13];
+    bool accept = false, stop = false;
+    if (F.first) {
+        F.first = 0;
+        accept = true;
+        F.cost = cq;
+    } else {
+        if (cq < F.cost) {
+            const double rel = (F.cost - cq) / fmax(F.cost, 1e-300);
+            for (int i = 0; i < 4; i++) F.p[i] = F.q[i];
+            accept = true;
+            F.cost = cq;
+            F.mu = fmax(F.mu * 0.3, 1e-12);
+            stop = rel < 1e-15 || F.tiny;
+        } else {
+            F.mu *= 10.0;
+            stop = F.mu > 1e12 || F.tiny;
+        }
+        stop = stop || ++F.it >= kFitIter;
+    }
+    if (stop) {
+        F.done = 1;
+        atomicSub(left, 1);
+        return;
+    }
+    if (accept) {
+        F.A[0] = (double) (nlen[b] / 2);  // the sum of 1 * 1
+        for (int e = 0; e < 9; e++) F.A[1 + e] = sh[e];
+        F.jr0 = sh[9];
+        for (int e = 0; e < 3; e++) F.A[10 + e] = sh[10 + e];
+    }
+    // damped step (J^T J + mu diag) d = -J^T r, projected on the bounds
+    const double mu = F.mu;
+    double p[4];
+    for (int i = 0; i < 4; i++) p[i] = F.p[i];
+    double A[4][4], g[4];
+    int e = 0;
+    for (int i = 0; i < 4; i++)
+        for (int j = i; j < 4; j++) {
+            A[i][j] = F.A[e];
+            A[j][i] = F.A[e];
+            e++;
+        }
+    g[0] = -F.jr0;
+    for (int i = 1; i < 4; i++) g[i] = -F.A[9 + i];
+    for (int i = 0; i < 4; i++) A[i][i] += mu * (A[i][i] > 0.0 ? A[i][i] : 1.0);
+    // active set: a parameter on a bound whose descent direction points
+    // outside stays fixed (its row and column leave the system)
+    for (int i = 0; i < 4; i++) {
+        const bool act = (p[i] <= lo[i] && g[i] < 0.0) || (p[i] >= hi[i] && g[i] > 0.0);
+        if (act) {
+            for (int j = 0; j < 4; j++) {
+                A[i][j] = 0.0;
+                A[j][i] = 0.0;
+            }
+            A[i][i] = 1.0;
+            g[i] = 0.0;
+        }
+    }
+    // Gaussian elimination with partial pivoting (4x4)
+    for (int c = 0; c < 4; c++) {
+        int pr = c;
+        for (int r = c + 1; r < 4; r++)
+            if (fabs(A[r][c]) > fabs(A[pr][c])) pr = r;
+        for (int j = 0; j < 4; j++) {
+            const double t = A[c][j];
+            A[c][j] = A[pr][j];
+            A[pr][j] = t;
+        }
+        const double tg = g[c];
+        g[c] = g[pr];
+        g[pr] = tg;
+        for (int r = c + 1; r < 4; r++) {
+            const double fct = A[c][c] != 0.0 ? A[r][c] / A[c][c] : 0.0;
+            for (int j = c; j < 4; j++) A[r][j] -= fct * A[c][j];
+            g[r] -= fct * g[c];
+        }
+    }
+    double d[4];
+    for (int r = 3; r >= 0; r--) {
+        double v = g[r];
+        for (int j = r + 1; j < 4; j++) v -= A[r][j] * d[j];
+        d[r] = A[r][r] != 0.0 ? v / A[r][r] : 0.0;
+    }
+    double dn = 0.0, pn = 0.0;
+    for (int i = 0; i < 4; i++) {
+        const double q = fmin(fmax(p[i] + d[i], lo[i]), hi[i]);
+        F.q[i] = q;
+        dn += (q - p[i]) * (q - p[i]);
+        pn += p[i] * p[i];
+    }
+    F.tiny = sqrt(dn) <= 1e-14 * (sqrt(pn) + 1e-14) ? 1 : 0;
+}
+
+// psdm1 of the fitted model on rfftfreq(n), extended to the full even sequence
+// of length n (each value computed once and written to both its places)
+__global__ void k_psdm1_even(const FitState *__restrict__ st, const int *__restrict__ blocks,
+                             const int *__restrict__ nlen, int64_t nmax, int batch, double fsamp,
+                             double *__restrict__ out) {
     const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= nmax * batch) return;
-    const int64_t b = gid / nmax, t = gid % nmax;
+    const int64_t half = nmax / 2 + 1;
+    if (gid >= half * batch) return;
+    const int64_t b = gid / half, k = gid % half;
     const int64_t n = nlen[b];
-    if (t >= n) return;
-    const int64_t k = t <= n / 2 ? t : n - t;
-    const double *p = params + 4 * b;
+    if (k > n / 2) return;
+    const double *p = st[blocks[b]].p;
     const double f = (double) k * fsamp / (double) n;
     const double u = (f + p[3]) / p[2];
-    out[b * nmax + t] = pow(10.0, -p[0]) / (1.0 + pow(u, p[1]));
+    const double v = pow(10.0, -p[0]) / (1.0 + pow(u, p[1]));
+    out[b * nmax + k] = v;
+    if (k > 0 && n - k > n / 2) out[b * nmax + n - k] = v;
 }
 
 // invtt row: window[j] * Re(DFT(psdm1_even))[j] / n for j < lambda
-__global__ void k_invtt_rows(const double2 *__restrict__ X, const int *__restrict__ nlen, int64_t nout_max,
+__global__ void k_invtt_rows(const double2 *__restrict__ X, int64_t stride, const int *__restrict__ nlen,
                              const int *__restrict__ blocks, int batch, int lambda,
                              const double *__restrict__ window, double *__restrict__ invtt) {
     const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= (int64_t) lambda * batch) return;
     const int64_t b = gid / lambda, j = gid % lambda;
-    invtt[(int64_t) blocks[b] * lambda + j] = window[j] * (X[b * nout_max + j].x / (double) nlen[b]);
+    invtt[(int64_t) blocks[b] * lambda + j] = window[j] * (X[b * stride + j].x / (double) nlen[b]);
 }
 
 }  // namespace
@@ -486,13 +650,27 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
     MGPU_ARG(window_kind == MGPU_APOD_CHEBWIN || window_kind == MGPU_APOD_GAUSSIAN, "unknown window %d",
              window_kind);
     const std::vector<double> &win = apod_window(lambda, window_kind);
-    double *d_win, *d_params;
-    int64_t *d_start;
+    // every block's log periodogram, transform group by group; one fit of all of
+    // them; then the rows, group by group again
+    std::vector<int64_t> yoff((size_t) nb + 1, 0);
+    for (int b = 0; b < nb; b++) yoff[b + 1] = yoff[b] + block_sizes[b] / 2 + 1;
+    double *d_win, *d_y, *d_parts;
+    int64_t *d_start, *d_yoff;
+    int *d_len, *d_left;
+    FitState *d_fit;
     MGPU_RET(pb.arena.alloc(&d_win, (size_t) lambda));
-    MGPU_RET(pb.arena.alloc(&d_params, (size_t) 4 * nb));
     MGPU_RET(pb.arena.alloc(&d_start, (size_t) nb + 1));
+    MGPU_RET(pb.arena.alloc(&d_yoff, (size_t) nb + 1));
+    MGPU_RET(pb.arena.alloc(&d_len, (size_t) nb));
+    MGPU_RET(pb.arena.alloc(&d_left, 1));
+    MGPU_RET(pb.arena.alloc(&d_y, (size_t) yoff[nb]));
+    MGPU_RET(pb.arena.alloc(&d_fit, (size_t) nb));
+    const int fit_run = std::min(nb, 1 << 14);  // blocks evaluated by one launch (28 KB of chains each)
+    MGPU_RET(pb.arena.alloc(&d_parts, (size_t) fit_run * kFitSums * kChains));
     MGPU_HIP(hipMemcpyAsync(d_win, win.data(), sizeof(double) * lambda, hipMemcpyHostToDevice, s));
     MGPU_HIP(hipMemcpyAsync(d_start, start.data(), sizeof(int64_t) * (nb + 1), hipMemcpyHostToDevice, s));
+    MGPU_HIP(hipMemcpyAsync(d_yoff, yoff.data(), sizeof(int64_t) * (nb + 1), hipMemcpyHostToDevice, s));
+    MGPU_HIP(hipMemcpyAsync(d_len, block_sizes, sizeof(int) * nb, hipMemcpyHostToDevice, s));
     // group blocks by transform size (power of two n, or the Bluestein size)
     std::map<std::pair<int, int>, std::vector<int>> groups;  // (logm, pow2) -> blocks
     for (int b = 0; b < nb; b++) {
@@ -502,69 +680,104 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
         while (((int64_t) 1 << logm) < (p2 ? n : 2 * n - 1)) logm++;
         groups[{logm, p2 ? 1 : 0}].push_back(b);
     }
-    for (auto &kv : groups) {
-        const int logm = kv.first.first;
-        const bool p2 = kv.first.second != 0;
-        const std::vector<int> &bl = kv.second;
-        // batches bounded to ~2 GiB of complex work per buffer
-        const int64_t M = (int64_t) 1 << logm;
-        const int per = (int) std::max<int64_t>(1, ((int64_t) 1 << 27) / M);
-        for (size_t g0 = 0; g0 < bl.size(); g0 += (size_t) per) {
-            const int batch = (int) std::min<size_t>((size_t) per, bl.size() - g0);
-            std::vector<int> blk(bl.begin() + g0, bl.begin() + g0 + batch), nlen((size_t) batch);
-            std::vector<int64_t> xoff((size_t) batch);
-            int64_t nmax = 0, tot = 0;
-            for (int i = 0; i < batch; i++) {
-                nlen[i] = block_sizes[blk[i]];
-                nmax = std::max<int64_t>(nmax, nlen[i]);
+    for (int pass = 0; pass < 2; pass++) {
+        if (pass == 1) {
+            k_fit_init<<<grid_for(nb, 256), 256, 0, s>>>(d_fit, nb);
+            MGPU_LAUNCHED();
+            int left = nb;
+            MGPU_HIP(hipMemcpyAsync(d_left, &left, sizeof(int), hipMemcpyHostToDevice, s));
+            // an evaluation and a decision a step, kFitIter of them after the first at
+            // most; the host looks every kFitPoll steps whether a block is left
+            constexpr int kFitPoll = 8;
+            for (int it = 0; it <= kFitIter && left > 0; it++) {
+                for (int b0 = 0; b0 < nb; b0 += fit_run) {
+                    const unsigned n = (unsigned) std::min(fit_run, nb - b0);
+                    k_fit_eval<<<n * kChainGroups, kChainWG, 0, s>>>(d_y, d_yoff + b0, d_len + b0, fsamp, d_fit + b0,
+                                                                     d_parts);
+                    MGPU_LAUNCHED();
+                    k_fit_step<<<n, 64 * kFitSums, 0, s>>>(d_parts, d_len + b0, d_fit + b0, d_left);
+                    MGPU_LAUNCHED();
+                }
+                if (it % kFitPoll == kFitPoll - 1) {
+                    MGPU_HIP(hipMemcpyAsync(&left, d_left, sizeof(int), hipMemcpyDeviceToHost, s));
+                    MGPU_HIP(hipStreamSynchronize(s));
+                }
             }
-            for (int i = 0; i < batch; i++) {
-                xoff[i] = tot;
-                tot += nmax;
+            if (h_params) {
+                std::vector<FitState> hf((size_t) nb);
+                MGPU_HIP(hipMemcpyAsync(hf.data(), d_fit, sizeof(FitState) * nb, hipMemcpyDeviceToHost, s));
+                MGPU_HIP(hipStreamSynchronize(s));
+                for (int b = 0; b < nb; b++)
+                    for (int k = 0; k < 4; k++) h_params[4 * (int64_t) b + k] = hf[b].p[k];
             }
-            int *d_blk, *d_nlen;
-            int64_t *d_xoff;
-            double *d_xw, *d_w2, *d_y, *d_even;
-            double2 *d_X;
-            MGPU_RET(pb.arena.alloc(&d_blk, (size_t) batch));
-            MGPU_RET(pb.arena.alloc(&d_nlen, (size_t) batch));
-            MGPU_RET(pb.arena.alloc(&d_xoff, (size_t) batch));
-            MGPU_RET(pb.arena.alloc(&d_xw, (size_t) tot));
-            MGPU_RET(pb.arena.alloc(&d_w2, (size_t) batch));
-            MGPU_RET(pb.arena.alloc(&d_y, (size_t) (nmax / 2 + 1) * batch));
-            MGPU_RET(pb.arena.alloc(&d_even, (size_t) tot));
-            MGPU_RET(pb.arena.alloc(&d_X, (size_t) tot));
-            MGPU_HIP(hipMemcpyAsync(d_blk, blk.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
-            MGPU_HIP(hipMemcpyAsync(d_nlen, nlen.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
-            MGPU_HIP(hipMemcpyAsync(d_xoff, xoff.data(), sizeof(int64_t) * batch, hipMemcpyHostToDevice, s));
-            MGPU_HIP(hipMemsetAsync(d_xw, 0, sizeof(double) * tot, s));
-            k_detrend_window<<<batch, 256, 0, s>>>(d_noise, d_start, d_nlen, d_blk, d_xoff, d_xw, d_w2);
-            MGPU_LAUNCHED();
-            MGPU_RET(dft_real(pb, d_xw, d_xoff, d_nlen, batch, logm, p2, nmax, d_X));
-            k_logpsd<<<grid_for((nmax / 2 + 1) * batch, 256), 256, 0, s>>>(d_X, d_nlen, nmax, batch, d_w2, fsamp, d_y);
-            MGPU_LAUNCHED();
-            k_fit<<<batch, 256, 0, s>>>(d_y, d_nlen, nmax, fsamp, d_params + 4 * (int64_t) 0 + 0);
-            MGPU_LAUNCHED();
-            // params of this batch were written at 4 * local index: move them to their blocks below
-            std::vector<double> hp((size_t) 4 * batch);
-            MGPU_HIP(hipMemcpyAsync(hp.data(), d_params, sizeof(double) * 4 * batch, hipMemcpyDeviceToHost, s));
-            MGPU_HIP(hipStreamSynchronize(s));
-            if (h_params)
-                for (int i = 0; i < batch; i++)
-                    for (int k = 0; k < 4; k++) h_params[4 * (int64_t) blk[i] + k] = hp[4 * (size_t) i + k];
-            k_psdm1_even<<<grid_for(tot, 256), 256, 0, s>>>(d_params, d_nlen, nmax, batch, fsamp, d_even);
-            MGPU_LAUNCHED();
-            MGPU_RET(dft_real(pb, d_even, d_xoff, d_nlen, batch, logm, p2, nmax, d_X));
-            k_invtt_rows<<<grid_for((int64_t) lambda * batch, 256), 256, 0, s>>>(d_X, d_nlen, nmax, d_blk, batch,
-                                                                                 lambda, d_win, d_invtt);
-            MGPU_LAUNCHED();
-            MGPU_HIP(hipStreamSynchronize(s));
-            for (void *p : {(void *) d_blk, (void *) d_nlen, (void *) d_xoff, (void *) d_xw, (void *) d_w2,
-                            (void *) d_y, (void *) d_even, (void *) d_X})
-                pb.arena.release(p);
+        }
+        for (auto &kv : groups) {
+            const int logm = kv.first.first;
+            const bool p2 = kv.first.second != 0;
+            const std::vector<int> &bl = kv.second;
+            // batches bounded to ~2 GiB of complex work per buffer
+            const int64_t M = (int64_t) 1 << logm;
+            const int per = (int) std::min<int64_t>(1 << 17, std::max<int64_t>(1, ((int64_t) 1 << 27) / M));
+            for (size_t g0 = 0; g0 < bl.size(); g0 += (size_t) per) {
+                const int batch = (int) std::min<size_t>((size_t) per, bl.size() - g0);
+                std::vector<int> blk(bl.begin() + g0, bl.begin() + g0 + batch), nlen((size_t) batch);
+                std::vector<int64_t> xoff((size_t) batch);
+                int64_t nmax = 0, tot = 0;
+                for (int i = 0; i < batch; i++) {
+                    nlen[i] = block_sizes[blk[i]];
+                    nmax = std::max<int64_t>(nmax, nlen[i]);
+                }
+                for (int i = 0; i < batch; i++) {
+                    xoff[i] = tot;
+                    tot += nmax;
+                }
+                int *d_blk, *d_nlen;
+                int64_t *d_xoff;
+                double *d_xw, *d_w2, *d_ps;
+                double2 *d_X = nullptr;
+                Dft dft(pb, logm, batch, p2, nmax);
+                MGPU_RET(dft.alloc());
+                MGPU_RET(pb.arena.alloc(&d_blk, (size_t) batch));
+                MGPU_RET(pb.arena.alloc(&d_nlen, (size_t) batch));
+                MGPU_RET(pb.arena.alloc(&d_xoff, (size_t) batch));
+                MGPU_RET(pb.arena.alloc(&d_xw, (size_t) tot));
+                MGPU_RET(pb.arena.alloc(&d_w2, (size_t) batch));
+                MGPU_RET(pb.arena.alloc(&d_ps, (size_t) 3 * kChains * batch));
+                if (!p2) MGPU_RET(pb.arena.alloc(&d_X, (size_t) tot));
+                MGPU_HIP(hipMemcpyAsync(d_blk, blk.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
+                MGPU_HIP(hipMemcpyAsync(d_nlen, nlen.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
+                MGPU_HIP(hipMemcpyAsync(d_xoff, xoff.data(), sizeof(int64_t) * batch, hipMemcpyHostToDevice, s));
+                const unsigned gc = (unsigned) batch * kChainGroups, gh = grid_for((nmax / 2 + 1) * batch, 256);
+                if (pass == 0) {
+                    double *wparts = d_ps + (size_t) 2 * kChains * batch;
+                    k_line_sums<<<gc, kChainWG, 0, s>>>(d_noise, d_start, d_nlen, d_blk, d_ps);
+                    MGPU_LAUNCHED();
+                    k_detrend_window<<<gc, kChainWG, 0, s>>>(d_noise, d_start, d_nlen, d_blk, d_xoff, d_ps, d_xw,
+                                                             wparts);
+                    MGPU_LAUNCHED();
+                    k_chain_tree<<<batch, 64, 0, s>>>(wparts, d_w2);
+                    MGPU_LAUNCHED();
+                    MGPU_RET(dft.run(d_xw, d_xoff, d_nlen, d_X));
+                    k_logpsd<<<gh, 256, 0, s>>>(dft.X, dft.stride, d_nlen, nmax, batch, d_w2, fsamp, d_blk, d_yoff,
+                                                d_y);
+                } else {
+                    k_psdm1_even<<<gh, 256, 0, s>>>(d_fit, d_blk, d_nlen, nmax, batch, fsamp, d_xw);
+                    MGPU_LAUNCHED();
+                    MGPU_RET(dft.run(d_xw, d_xoff, d_nlen, d_X));
+                    k_invtt_rows<<<grid_for((int64_t) lambda * batch, 256), 256, 0, s>>>(
+                            dft.X, dft.stride, d_nlen, d_blk, batch, lambda, d_win, d_invtt);
+                }
+                MGPU_LAUNCHED();
+                MGPU_HIP(hipStreamSynchronize(s));  // before the work buffers go back to the block cache
+                for (void *p : {(void *) d_blk, (void *) d_nlen, (void *) d_xoff, (void *) d_xw, (void *) d_w2,
+                                (void *) d_ps, (void *) d_X})
+                    if (p) pb.arena.release(p);
+            }
         }
     }
-    for (void *p : {(void *) d_win, (void *) d_params, (void *) d_start}) pb.arena.release(p);
+    for (void *p : {(void *) d_win, (void *) d_start, (void *) d_yoff, (void *) d_len, (void *) d_left, (void *) d_y,
+                    (void *) d_fit, (void *) d_parts})
+        pb.arena.release(p);
     return MGPU_OK;
 }
 
