@@ -474,6 +474,12 @@ struct TItem {           // one workgroup of T^T: a sweep, an azimuth bin or a t
     int64_t rel;         // first output amplitude, relative to the block's amplitudes
     int stride, pad;     // distance between the class outputs (sweeps or time bins)
 };
+struct TPieces {         // T^T's pieces of one CES: runs of samples of one sweep (or time bin) inside a chunk
+    int p0, h0;          // first sweep piece and first time-bin piece (numbered over all CES)
+    int np, nh;          // pieces of this CES
+    int ch0, nch;        // its chunks
+    int s0, q0;          // first entries of its sweeps and time bins in d_sw_piece / d_tb_piece
+};
 struct BTask {           // one kernel entry (and its mirror) summed in sample order
     int kind;            // 0 samples [lo, hi); 1 weighted, 2 unweighted over perm[lo, hi)
     int row, col;        // entry within the block
@@ -510,8 +516,23 @@ struct Templates {
     int64_t *d_boff = nullptr;              // [nb+1] first kernel entry of each block
     double *d_B = nullptr, *d_Binv = nullptr; // [nB] row-major nt_b x nt_b blocks
     double *d_a1 = nullptr, *d_a2 = nullptr;  // [ntot]
-    TItem *d_items = nullptr;
+    TItem *d_items = nullptr;               // azimuth bins summed on their own (more than kChunkBins of them)
     int nitems = 0;
+    // T^T in one pass over the samples (k_tmpl_part, k_tmpl_fin)
+    int nchunks = 0;
+    int *d_chunk_ces = nullptr, *d_chunk_lo = nullptr;      // [nchunks] CES and first CES sample of each chunk
+    int *d_chunk_p = nullptr, *d_chunk_h = nullptr;         // [nchunks + 1] first sweep / time-bin piece
+    int2 *d_ppiece = nullptr, *d_hpiece = nullptr;          // pieces: first CES sample, samples
+    int *d_sw_piece = nullptr, *d_tb_piece = nullptr;       // first piece of each sweep / time bin (one past the last too)
+    TPieces *d_pieces = nullptr;                            // [nces]
+    unsigned short *d_order = nullptr, *d_abin = nullptr;   // [ncs] chunk samples by azimuth bin; [nchunks * (nsss + 1)] bin starts
+    int64_t *d_poff = nullptr;                              // [nb] first partial of each block
+    double *d_part = nullptr;
+    // B^+ by CES: the representative block and each block's factor
+    int *d_rep_blk = nullptr, *d_row_ces = nullptr;         // [nces]; [nrows] CES of each row of a representative
+    int *d_row0 = nullptr;                                  // [nces] first of those rows
+    double *d_scale = nullptr;                              // [nb]
+    int nrows = 0;
     double build_ms = 0.0;
 };
 

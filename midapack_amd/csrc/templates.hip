@@ -16,10 +16,11 @@
 // MI355X layout.  Blocks span their CES (CES-major), so every per-sample table
 // (sweep, azimuth bin, Legendre and HWP weights, sample orders) is stored once
 // per CES and read by all its detectors from L2 / MALL.  Per PCG iteration:
-//   k_tmpl_tr   T^T: one workgroup per (block, sweep | azimuth bin | time bin),
-//               every class of the group accumulated in registers, fixed-order
-//               workgroup sums (deterministic);
-//   k_tmpl_binv a2 = B^+ a1: one wave per amplitude row, coalesced row reads;
+//   k_tmpl_part T^T over chunks of 2048 samples of a block, every class from one
+//               read of the samples; k_tmpl_fin adds the chunks' partial sums in
+//               a fixed order (deterministic);
+//   k_tmpl_binv a2 = B^+ a1: one wave per amplitude row of a CES, for all its
+//               detectors (their B^+ differ by a factor);
 //   k_tmpl_sub  y -= w_b T a2: one thread per CES sample looping over the CES's
 //               detectors, so each sample's weights are loaded once; the classes
 //               are added in class order exactly as TVecProd does.
@@ -74,84 +75,256 @@ __device__ __forceinline__ double wg_sum(double v, double *red) {
 // ---------------------------------------------------------------------------
 // kernels: PCG iteration
 // ---------------------------------------------------------------------------
-// T^T (s_b y): one workgroup per item (a sweep, azimuth bin or time bin of a
-// block; blocks in order, so the detectors of a CES follow each other and
-// reuse its table entries from L2 / MALL); kind 0 sums leg[o] * v over a
-// sweep for every order, kind 1 sums v over an azimuth bin (its samples listed
-// in the azimuth order), kind 2 sums hc[h] * v over a time bin for every HWP
-// slot, with v = s_b * y (s_b = T0[b], the weighting of apply_weights fused in;
-// 1 when scale is NULL)
-__global__ __launch_bounds__(kTW) void k_tmpl_tr(const TItem *__restrict__ items, const double *__restrict__ y,
-                                                 const double *__restrict__ scale,
-                                                 const int64_t *__restrict__ start, const int64_t *__restrict__ c0,
-                                                 int ndet, const int *__restrict__ perm_az,
-                                                 const double *__restrict__ leg, const double *__restrict__ hc,
-                                                 int64_t ncs, int npoly, int nh2, const int64_t *__restrict__ off,
-                                                 double *__restrict__ out, const int *__restrict__ state) {
-    __shared__ double red[kTW / 64];
-    if (state && *state) return;  // the solve has stopped: queued iterations do no work
-    const TItem it = items[blockIdx.x];
-    const int b = it.b;
-    const int64_t cb = c0[b / ndet];
-    const int nk = it.kind == 0 ? npoly : it.kind == 1 ? 1 : nh2;
-    const double *__restrict__ yb = y + start[b];
-    const double sc = scale ? scale[b] : 1.0;
-    double acc[kSlots];
+constexpr int kTChunk = 2048;    // samples of a T^T workgroup
+constexpr int kTPiece = 128;     // longest run of a sweep or time bin summed by 16 lanes
+constexpr int kChunkBins = 256;  // most azimuth bins that a chunk sorts its samples into
+
+__device__ __forceinline__ double sum16(double v) {
+    for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 16);
+    return v;
+}
+
+struct TrArgs {
+    const double *y, *scale;
+    const int64_t *start, *c0, *poff;
+    const int *len, *chunk_ces, *chunk_lo, *chunk_p, *chunk_h;
+    const int2 *ppiece, *hpiece;
+    const TPieces *pieces;
+    const unsigned short *order, *abin;
+    const double *leg, *hc;
+    int64_t ncs;
+    int ndet, nchunks, npoly, nh2, nsss;  // nsss 0: no azimuth class here
+    double *part;
+    const int *state;
+};
+
+// Partial sums of T^T (s_b y) over one chunk of one block.  The chunk's samples v
+// = s_b y (s_b = T0[b], the weighting of apply_weights fused in; 1 when scale is
+// NULL) go to LDS once; groups of 16 lanes then sum leg[o] v over its pieces of
+// sweeps, hc[h] v over its pieces of time bins and v over its azimuth bins (the
+// samples in the chunk's azimuth order).  Detectors of a chunk run together on
+// one XCD, which keeps the chunk's tables in its L2.  Bound by latency (87 % of
+// the waves' cycles wait): on 32 blocks of 2^18 samples 48 us and 5.5 us for
+// k_tmpl_fin, where a workgroup per sweep and bin, which read the samples once
+// per class, took 101 us.  (Four detectors a workgroup, for fewer loads of the
+// weights, leave fewer waves to hide it: 61 us.)
+template <int NP, int NH>
+__global__ __launch_bounds__(256) void k_tmpl_part(TrArgs a) {
+    if (a.state && *a.state) return;  // the solve has stopped: queued iterations do no work
+    __shared__ double sv[kTChunk];
+    // workgroup b runs on XCD b % 8: each XCD gets a contiguous run of (chunk, detector)
+    const int n_all = a.nchunks * a.ndet, x = (int) blockIdx.x & 7, rem = n_all & 7;
+    const int idx = x * (n_all >> 3) + min(x, rem) + ((int) blockIdx.x >> 3);
+    const int chunk = idx / a.ndet, c = a.chunk_ces[chunk], b = c * a.ndet + idx % a.ndet, lo = a.chunk_lo[chunk];
+    const int n = min(kTChunk, a.len[c] - lo);
+    const int64_t cb = a.c0[c];
+    const double sc = a.scale ? a.scale[b] : 1.0;
+    const double *__restrict__ yb = a.y + a.start[b] + lo;
 #pragma unroll
-    for (int k = 0; k < kSlots; k++) acc[k] = 0.0;
-    if (it.kind == 0) {
-        for (int i = it.lo + (int) threadIdx.x; i < it.hi; i += kTW) {
-            const double v = sc * yb[i];
-#pragma unroll
-            for (int k = 0; k < kSlots; k++)
-                if (k < npoly) acc[k] += leg[(int64_t) k * ncs + cb + i] * v;
-        }
-    } else if (it.kind == 1) {
-        for (int i = it.lo + (int) threadIdx.x; i < it.hi; i += kTW) acc[0] += sc * yb[perm_az[cb + i]];
-    } else {
-        for (int i = it.lo + (int) threadIdx.x; i < it.hi; i += kTW) {
-            const double v = sc * yb[i];
-#pragma unroll
-            for (int k = 0; k < kSlots; k++)
-                if (k < nh2) acc[k] += hc[(int64_t) k * ncs + cb + i] * v;
-        }
+    for (int k = 0; k < kTChunk / 256; k++) {
+        const int i = (int) threadIdx.x + k * 256;
+        if (i < n) sv[i] = sc * yb[i];
     }
-    const int64_t o = off[b] + it.rel;
+    __syncthreads();
+    const int lane = threadIdx.x & 15;
+    const TPieces P = a.pieces[c];
+    double *__restrict__ op = a.part + a.poff[b], *__restrict__ oh = op + (int64_t) a.npoly * P.np;
+    double *__restrict__ oa = oh + (int64_t) a.nh2 * P.nh + (int64_t) (chunk - P.ch0) * a.nsss;
+    const int p0 = a.chunk_p[chunk], np = a.chunk_p[chunk + 1] - p0, h0 = a.chunk_h[chunk],
+              nh = a.chunk_h[chunk + 1] - h0;
+    for (int k = threadIdx.x >> 4; k < np + nh + a.nsss; k += 16) {
+        if (k < np) {
+            const int2 pc = a.ppiece[p0 + k];
+            const double *__restrict__ w = a.leg + cb + pc.x, *v = sv + (pc.x - lo);
+            double acc[NP];
 #pragma unroll
-    for (int k = 0; k < kSlots; k++) {
-        if (k >= nk) break;
-        const double s = wg_sum(acc[k], red);
-        if (threadIdx.x == 0) out[o + (int64_t) k * it.stride] = s;
+            for (int o = 0; o < NP; o++) acc[o] = 0.0;
+#pragma unroll 4
+            for (int i = lane; i < pc.y; i += 16)
+#pragma unroll
+                for (int o = 0; o < NP; o++)
+                    if (o < a.npoly) acc[o] += w[o * a.ncs + i] * v[i];
+#pragma unroll
+            for (int o = 0; o < NP; o++) {
+                const double s = sum16(acc[o]);
+                if (o < a.npoly && lane == 0) op[(int64_t) (p0 - P.p0 + k) * a.npoly + o] = s;
+            }
+        } else if (k < np + nh) {
+            const int2 pc = a.hpiece[h0 + k - np];
+            const double *__restrict__ w = a.hc + cb + pc.x, *v = sv + (pc.x - lo);
+            double acc[NH];
+#pragma unroll
+            for (int h = 0; h < NH; h++) acc[h] = 0.0;
+#pragma unroll 4
+            for (int i = lane; i < pc.y; i += 16)
+#pragma unroll
+                for (int h = 0; h < NH; h++)
+                    if (h < a.nh2) acc[h] += w[h * a.ncs + i] * v[i];
+#pragma unroll
+            for (int h = 0; h < NH; h++) {
+                const double s = sum16(acc[h]);
+                if (h < a.nh2 && lane == 0) oh[(int64_t) (h0 - P.h0 + k - np) * a.nh2 + h] = s;
+            }
+        } else {
+            const int q = k - np - nh;
+            const unsigned short *__restrict__ ab = a.abin + (int64_t) chunk * (a.nsss + 1) + q;
+            const unsigned short *__restrict__ ord = a.order + cb + lo;
+            const int e = ab[1];
+            double acc = 0.0;
+#pragma unroll 4
+            for (int i = ab[0] + lane; i < e; i += 16) acc += sv[ord[i]];
+            acc = sum16(acc);
+            if (lane == 0) oa[q] = acc;
+        }
     }
 }
 
-// a2 = B^+ a1, one wave per amplitude row
+// T^T amplitudes from the chunks' partial sums, 16 lanes an amplitude
+__global__ __launch_bounds__(256) void k_tmpl_fin(const double *__restrict__ part, const int64_t *__restrict__ poff,
+                                                  const TPieces *__restrict__ pieces,
+                                                  const int *__restrict__ sw_piece, const int *__restrict__ tb_piece,
+                                                  const int *__restrict__ ns_c, const int *__restrict__ nh_c,
+                                                  const int *__restrict__ row_block, const int64_t *__restrict__ off,
+                                                  int64_t ntot, int ndet, int npoly, int nh2, int nsss, int az_here,
+                                                  double *__restrict__ out, const int *__restrict__ state) {
+    if (state && *state) return;
+    const int64_t r = ((int64_t) blockIdx.x * 256 + threadIdx.x) >> 4;
+    if (r >= ntot) return;  // uniform over the 16 lanes
+    const int lane = threadIdx.x & 15, b = row_block[r], c = b / ndet;
+    const TPieces P = pieces[c];
+    const int ns = ns_c[c], nh = nh_c[c];
+    int l = (int) (r - off[b]), e0, e1;
+    int64_t step;
+    const double *__restrict__ p = part + poff[b];
+    if (l < npoly * ns) {
+        const int s = P.s0 + l % ns;
+        e0 = sw_piece[s] - P.p0;
+        e1 = sw_piece[s + 1] - P.p0;
+        step = npoly;
+        p += l / ns;
+    } else if ((l -= npoly * ns) < nsss) {
+        if (!az_here) return;
+        e0 = 0;
+        e1 = P.nch;
+        step = nsss;
+        p += (int64_t) npoly * P.np + (int64_t) nh2 * P.nh + l;
+    } else {
+        l -= nsss;
+        const int q = P.q0 + l % nh;
+        e0 = tb_piece[q] - P.h0;
+        e1 = tb_piece[q + 1] - P.h0;
+        step = nh2;
+        p += (int64_t) npoly * P.np + l / nh;
+    }
+    double acc = 0.0;
+#pragma unroll 4
+    for (int e = e0 + lane; e < e1; e += 16) acc += p[e * step];
+    acc = sum16(acc);
+    if (lane == 0) out[r] = acc;
+}
+
+// samples of every chunk by azimuth bin (stable), and where each bin starts
+__global__ __launch_bounds__(256) void k_chunk_order(const int *__restrict__ az, const int64_t *__restrict__ c0,
+                                                     const int *__restrict__ len, const int *__restrict__ chunk_ces,
+                                                     const int *__restrict__ chunk_lo, int nsss,
+                                                     unsigned short *__restrict__ order,
+                                                     unsigned short *__restrict__ abin) {
+    __shared__ unsigned short sa[kTChunk];
+    __shared__ unsigned short cnt[kChunkBins + 1];
+    const int c = chunk_ces[blockIdx.x], lo = chunk_lo[blockIdx.x], n = min(kTChunk, len[c] - lo);
+    const int64_t g = c0[c] + lo;
+    const int t = threadIdx.x;
+    for (int i = t; i < n; i += 256) sa[i] = (unsigned short) az[g + i];
+    __syncthreads();
+    int k = 0;
+    if (t < nsss) {
+        for (int i = 0; i < n; i++) k += sa[i] == t;
+        cnt[t + 1] = (unsigned short) k;
+    }
+    if (t == 0) cnt[0] = 0;
+    __syncthreads();
+    if (t == 0)
+        for (int q = 0; q < nsss; q++) cnt[q + 1] = (unsigned short) (cnt[q + 1] + cnt[q]);
+    __syncthreads();
+    if (t < nsss) {
+        int o = cnt[t];
+        for (int i = 0; i < n; i++)
+            if (sa[i] == t) order[g + o++] = (unsigned short) i;
+    }
+    for (int q = t; q <= nsss; q += 256) abin[(int64_t) blockIdx.x * (nsss + 1) + q] = cnt[q];
+}
+
+// azimuth amplitudes where the bins are too many for a chunk to sort its samples
+// into (kChunkBins): one workgroup per bin of a block sums s_b y over the bin's
+// samples, listed in the azimuth order
+__global__ __launch_bounds__(kTW) void k_tmpl_az(const TItem *__restrict__ items, const double *__restrict__ y,
+                                                 const double *__restrict__ scale,
+                                                 const int64_t *__restrict__ start, const int64_t *__restrict__ c0,
+                                                 int ndet, const int *__restrict__ perm_az,
+                                                 const int64_t *__restrict__ off, double *__restrict__ out,
+                                                 const int *__restrict__ state) {
+    __shared__ double red[kTW / 64];
+    if (state && *state) return;
+    const TItem it = items[blockIdx.x];
+    const int b = it.b;
+    const int64_t cb = c0[b / ndet];
+    const double *__restrict__ yb = y + start[b];
+    const double sc = scale ? scale[b] : 1.0;
+    double acc = 0.0;
+    for (int i = it.lo + (int) threadIdx.x; i < it.hi; i += kTW) acc += sc * yb[perm_az[cb + i]];
+    const double s = wg_sum(acc, red);
+    if (threadIdx.x == 0) out[off[b] + it.rel] = s;
+}
+
+// a2 = B^+ a1.  B_b^+ = scale[b] B_r^+ for the blocks b of a CES with
+// representative r, so one wave per row of B_r^+ serves all detectors, eight at a
+// time: on 4 CES x 8 detectors of 672 amplitudes 14 MB are read instead of 115 MB
+// (34 us at 3.4 TB/s -> 17.5 us, bound by the reads of a1 from L2).
 __global__ __launch_bounds__(256) void k_tmpl_binv(const double *__restrict__ Binv, const int64_t *__restrict__ boff,
-                                                   const int64_t *__restrict__ off,
-                                                   const int *__restrict__ row_block, int64_t ntot,
+                                                   const int64_t *__restrict__ off, const int *__restrict__ rep_blk,
+                                                   const int *__restrict__ row_ces, const int *__restrict__ row0,
+                                                   int nrows, int ndet, const double *__restrict__ scale,
                                                    const double *__restrict__ a1, double *__restrict__ a2,
                                                    const int *__restrict__ state) {
     if (state && *state) return;
-    const int64_t r = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= ntot) return;  // uniform per wave
-    const int lane = threadIdx.x & 63;
-    const int b = row_block[r];
-    const int64_t o = off[b];
-    const int nt = (int) (off[b + 1] - o);
-    const double *__restrict__ row = Binv + boff[b] + (r - o) * nt;
-    double s = 0.0;
-    for (int k = lane; k < nt; k += 64) s += row[k] * a1[o + k];
-    s = wave_sum(s);
-    if (lane == 0) a2[r] = s;
+    constexpr int D = 8;
+    const int w = (int) blockIdx.x * 4 + (int) (threadIdx.x >> 6);
+    if (w >= nrows) return;  // uniform per wave
+    const int lane = threadIdx.x & 63, c = row_ces[w], r = w - row0[c], b0 = c * ndet;
+    const int64_t o0 = off[b0];
+    const int nt = (int) (off[b0 + 1] - o0);
+    const double *__restrict__ row = Binv + boff[rep_blk[c]] + (int64_t) r * nt;
+    for (int j0 = 0; j0 < ndet; j0 += D) {
+        const double *__restrict__ v[D];  // the CES's blocks have nt amplitudes each, one after the other
+#pragma unroll
+        for (int d = 0; d < D; d++) v[d] = a1 + o0 + (int64_t) min(j0 + d, ndet - 1) * nt;
+        double s[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) s[d] = 0.0;
+#pragma unroll 2
+        for (int k = lane; k < nt; k += 64) {
+            const double m = row[k];
+#pragma unroll
+            for (int d = 0; d < D; d++) s[d] += m * v[d][k];
+        }
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const double t = wave_sum(s[d]);
+            if (lane == 0 && j0 + d < ndet) a2[o0 + (int64_t) (j0 + d) * nt + r] = scale[b0 + j0 + d] * t;
+        }
+    }
 }
 
 // y[t] = v[t] - w_b (T a2)[t], v = in_scale_b q (the fused apply_weights) or q,
 // for every detector of the CES at CES sample i; the classes are added to 0 in
 // class order (TVecProd), then scaled by w_b (apply_weights) and subtracted
-// (pcg_true.c:453-454).  INPLACE: q is y.
-template <bool INPLACE>
-__global__ __launch_bounds__(256) void k_tmpl_sub(const double *__restrict__ q, const double *__restrict__ in_scale,
-                                                  double *__restrict__ y, const int64_t *__restrict__ start,
+// (pcg_true.c:453-454).  INPLACE: q is y.  NP, NH: npoly and nh2 at most.  Four
+// detectors at a time keep their loads in flight together (bound by HBM: 16 B a
+// sample; 32 blocks of 2^18 samples, one detector at a time with 16 + 16 class
+// slots: 70 us, now 40 us).
+template <bool INPLACE, int NP, int NH>
+__global__ __launch_bounds__(256) void k_tmpl_sub(const double *q, const double *__restrict__ in_scale, double *y,
+                                                  const int64_t *__restrict__ start,
                                                   const double *__restrict__ T0, int ndet,
                                                   const int64_t *__restrict__ c0, const int *__restrict__ ns_c,
                                                   const int *__restrict__ nh_c, const int *__restrict__ sweep,
@@ -167,36 +340,44 @@ __global__ __launch_bounds__(256) void k_tmpl_sub(const double *__restrict__ q, 
     if (i >= len[c]) return;
     const int ns = ns_c[c], nh = nh_c[c];
     const int s = npoly ? sweep[g] : -1;
-    double wl[kSlots], wh[kSlots];
+    double wl[NP], wh[NH];
 #pragma unroll
-    for (int k = 0; k < kSlots; k++) {
-        wl[k] = (k < npoly && s >= 0) ? leg[(int64_t) k * ncs + g] : 0.0;
-        wh[k] = k < nh2 ? hc[(int64_t) k * ncs + g] : 0.0;
-    }
+    for (int k = 0; k < NP; k++) wl[k] = (k < npoly && s >= 0) ? leg[(int64_t) k * ncs + g] : 0.0;
+#pragma unroll
+    for (int k = 0; k < NH; k++) wh[k] = k < nh2 ? hc[(int64_t) k * ncs + g] : 0.0;
     const int a = ground ? az[g] : 0;
     const int tb = nh2 ? (int) floor((double) i / fsdt) : 0;
-    const double *__restrict__ src = INPLACE ? y : q;
-    for (int j = 0; j < ndet; j++) {
-        const int b = c * ndet + j;
-        int64_t base = off[b];
-        double r = 0.0;
-        if (s >= 0) {
+    const double *src = INPLACE ? y : q;
+    constexpr int D = 4;
+    for (int j0 = 0; j0 < ndet; j0 += D) {
+        double v[D], r[D];
 #pragma unroll
-            for (int k = 0; k < kSlots; k++)
-                if (k < npoly) r += wl[k] * a2[base + (int64_t) k * ns + s];
-        }
-        base += (int64_t) npoly * ns;
-        if (ground) {
-            r += a2[base + a];
-            base += nsss;
+        for (int d = 0; d < D; d++) {
+            const int b = c * ndet + min(j0 + d, ndet - 1);
+            v[d] = src[start[b] + i];
+            int64_t base = off[b];
+            r[d] = 0.0;
+            if (s >= 0) {
+#pragma unroll
+                for (int k = 0; k < NP; k++)
+                    if (k < npoly) r[d] += wl[k] * a2[base + (int64_t) k * ns + s];
+            }
+            base += (int64_t) npoly * ns;
+            if (ground) {
+                r[d] += a2[base + a];
+                base += nsss;
+            }
+#pragma unroll
+            for (int k = 0; k < NH; k++)
+                if (k < nh2) r[d] += wh[k] * a2[base + (int64_t) k * nh + tb];
         }
 #pragma unroll
-        for (int k = 0; k < kSlots; k++)
-            if (k < nh2) r += wh[k] * a2[base + (int64_t) k * nh + tb];
-        const int64_t t = start[b] + i;
-        const double tv = T0[b] * r;
-        const double v = in_scale ? in_scale[b] * src[t] : src[t];
-        y[t] = v - tv;
+        for (int d = 0; d < D; d++) {
+            if (j0 + d >= ndet) break;
+            const int b = c * ndet + j0 + d;
+            const double tv = T0[b] * r[d];
+            y[start[b] + i] = (in_scale ? in_scale[b] * v[d] : v[d]) - tv;
+        }
     }
 }
 
@@ -656,26 +837,77 @@ int templates_build(Problem &pb, const mgpu_templates *t) {
     std::vector<int> row_block((size_t) std::max<int64_t>(M.ntot, 1), 0);
     for (int b = 0; b < nb; b++)
         for (int64_t r = M.h_off[b]; r < M.h_off[b + 1]; r++) row_block[r] = b;
-    // T^T items of every block in block order: sweeps, azimuth bins, time bins
-    // (rel: the output offset inside the block's amplitudes)
-    std::vector<TItem> items;
-    for (int b = 0; b < nb; b++) {
-        const CesTables &C = ct[b / ndet];
-        if (M.npoly)
-            for (int sw = 0; sw < C.ns; sw++) items.push_back(TItem{b, 0, C.stamps[sw], C.stamps[sw + 1], sw, C.ns, 0});
-        if (M.ground) {
-            // azimuth bin a occupies a contiguous range of the azimuth order
-            int k = 0;
-            for (int a = 0; a < M.nsss; a++) {
-                int e = k;
-                while (e < C.len && C.az[C.perm[0][e]] == a) e++;
-                items.push_back(TItem{b, 1, k, e, (int64_t) M.npoly * C.ns + a, 0, 0});
-                k = e;
+    // T^T: chunks of kTChunk samples of every CES, and the pieces of its sweeps and
+    // time bins inside them (numbered in sample order over all CES)
+    const bool az_chunks = M.ground && M.nsss <= kChunkBins;
+    std::vector<int> chunk_ces, chunk_lo, chunk_p, chunk_h, sw_piece, tb_piece;
+    std::vector<int2> ppiece, hpiece;
+    std::vector<TPieces> pieces((size_t) nces);
+    std::vector<int64_t> poff((size_t) nb + 1, 0);
+    for (int c = 0; c < nces; c++) {
+        const CesTables &C = ct[c];
+        TPieces &P = pieces[c];
+        P.p0 = (int) ppiece.size();
+        P.h0 = (int) hpiece.size();
+        P.ch0 = (int) chunk_ces.size();
+        P.s0 = (int) sw_piece.size();
+        P.q0 = (int) tb_piece.size();
+        auto cut = [](std::vector<int2> &out, int lo, int hi) {
+            while (lo < hi) {
+                const int e = std::min({hi, lo + kTPiece, (lo / kTChunk + 1) * kTChunk});
+                out.push_back(make_int2(lo, e - lo));
+                lo = e;
             }
+        };
+        for (int sw = 0; M.npoly && sw < C.ns; sw++) {
+            sw_piece.push_back((int) ppiece.size());
+            cut(ppiece, C.stamps[sw], C.stamps[sw + 1]);
         }
-        if (nh2)
-            for (int q = 0; q < C.nh; q++)
-                items.push_back(TItem{b, 2, C.tbs[q], C.tbs[q + 1], (int64_t) M.npoly * C.ns + M.nsss + q, C.nh, 0});
+        sw_piece.push_back((int) ppiece.size());
+        for (int q = 0; nh2 && q < C.nh; q++) {
+            tb_piece.push_back((int) hpiece.size());
+            cut(hpiece, C.tbs[q], C.tbs[q + 1]);
+        }
+        tb_piece.push_back((int) hpiece.size());
+        int kp = P.p0, kh = P.h0;
+        for (int lo = 0; lo < C.len; lo += kTChunk) {
+            chunk_ces.push_back(c);
+            chunk_lo.push_back(lo);
+            chunk_p.push_back(kp);
+            chunk_h.push_back(kh);
+            while (kp < (int) ppiece.size() && ppiece[kp].x < lo + kTChunk) kp++;
+            while (kh < (int) hpiece.size() && hpiece[kh].x < lo + kTChunk) kh++;
+        }
+        P.np = (int) ppiece.size() - P.p0;
+        P.nh = (int) hpiece.size() - P.h0;
+        P.nch = (int) chunk_ces.size() - P.ch0;
+        for (int j = 0; j < ndet; j++) {
+            const int bb = c * ndet + j;
+            poff[bb + 1] = poff[bb] + (int64_t) M.npoly * P.np + (int64_t) nh2 * P.nh +
+                           (az_chunks ? (int64_t) P.nch * M.nsss : 0);
+        }
+    }
+    M.nchunks = (int) chunk_ces.size();
+    chunk_p.push_back((int) ppiece.size());
+    chunk_h.push_back((int) hpiece.size());
+    MGPU_ARG((int64_t) M.nchunks * ndet < INT32_MAX, "%d chunks of %d detectors are too many", M.nchunks, ndet);
+    std::vector<int> row_ces, row0((size_t) nces);
+    for (int c = 0; c < nces; c++) {
+        row0[c] = (int) row_ces.size();
+        row_ces.insert(row_ces.end(), (size_t) M.h_nt[(size_t) c * ndet], c);
+    }
+    M.nrows = (int) row_ces.size();
+    // azimuth bins summed on their own (rel: the output offset inside the block's amplitudes)
+    std::vector<TItem> items;
+    for (int b = 0; b < nb && M.ground && !az_chunks; b++) {
+        const CesTables &C = ct[b / ndet];
+        int k = 0;
+        for (int a = 0; a < M.nsss; a++) {  // bin a occupies a contiguous range of the azimuth order
+            int e = k;
+            while (e < C.len && C.az[C.perm[0][e]] == a) e++;
+            items.push_back(TItem{b, 1, k, e, (int64_t) M.npoly * C.ns + a, 0, 0});
+            k = e;
+        }
     }
     M.nitems = (int) items.size();
     MGPU_RET(pb.arena.alloc(&M.d_ns, (size_t) nces));
@@ -697,6 +929,26 @@ int templates_build(Problem &pb, const mgpu_templates *t) {
     MGPU_RET(pb.arena.alloc(&M.d_items, (size_t) std::max(1, M.nitems)));
     MGPU_RET(pb.arena.alloc(&M.d_ces_of, ces_of.size()));
     M.nwg_samples = (int) ces_of.size();
+    auto room = [](size_t n) { return std::max<size_t>(n, 1); };
+    MGPU_RET(pb.arena.alloc(&M.d_chunk_ces, room(chunk_ces.size())));
+    MGPU_RET(pb.arena.alloc(&M.d_chunk_lo, room(chunk_lo.size())));
+    MGPU_RET(pb.arena.alloc(&M.d_chunk_p, chunk_p.size()));
+    MGPU_RET(pb.arena.alloc(&M.d_chunk_h, chunk_h.size()));
+    MGPU_RET(pb.arena.alloc(&M.d_ppiece, room(ppiece.size())));
+    MGPU_RET(pb.arena.alloc(&M.d_hpiece, room(hpiece.size())));
+    MGPU_RET(pb.arena.alloc(&M.d_sw_piece, sw_piece.size()));
+    MGPU_RET(pb.arena.alloc(&M.d_tb_piece, tb_piece.size()));
+    MGPU_RET(pb.arena.alloc(&M.d_pieces, pieces.size()));
+    MGPU_RET(pb.arena.alloc(&M.d_poff, poff.size()));
+    MGPU_RET(pb.arena.alloc(&M.d_part, room((size_t) poff[nb])));
+    MGPU_RET(pb.arena.alloc(&M.d_rep_blk, (size_t) nces));
+    MGPU_RET(pb.arena.alloc(&M.d_row0, (size_t) nces));
+    MGPU_RET(pb.arena.alloc(&M.d_row_ces, room(row_ces.size())));
+    MGPU_RET(pb.arena.alloc(&M.d_scale, (size_t) nb));
+    if (az_chunks) {
+        MGPU_RET(pb.arena.alloc(&M.d_order, (size_t) ncs));
+        MGPU_RET(pb.arena.alloc(&M.d_abin, (size_t) M.nchunks * (M.nsss + 1)));
+    }
     auto up = [&](void *d, const void *h, size_t bytes) -> int {
         MGPU_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
         return MGPU_OK;
@@ -715,6 +967,23 @@ int templates_build(Problem &pb, const mgpu_templates *t) {
     MGPU_RET(up(M.d_row_block, row_block.data(), sizeof(int) * row_block.size()));
     if (!items.empty()) MGPU_RET(up(M.d_items, items.data(), sizeof(TItem) * items.size()));
     MGPU_RET(up(M.d_ces_of, ces_of.data(), sizeof(int) * ces_of.size()));
+    MGPU_RET(up(M.d_chunk_ces, chunk_ces.data(), sizeof(int) * chunk_ces.size()));
+    MGPU_RET(up(M.d_chunk_lo, chunk_lo.data(), sizeof(int) * chunk_lo.size()));
+    MGPU_RET(up(M.d_chunk_p, chunk_p.data(), sizeof(int) * chunk_p.size()));
+    MGPU_RET(up(M.d_chunk_h, chunk_h.data(), sizeof(int) * chunk_h.size()));
+    if (!ppiece.empty()) MGPU_RET(up(M.d_ppiece, ppiece.data(), sizeof(int2) * ppiece.size()));
+    if (!hpiece.empty()) MGPU_RET(up(M.d_hpiece, hpiece.data(), sizeof(int2) * hpiece.size()));
+    MGPU_RET(up(M.d_sw_piece, sw_piece.data(), sizeof(int) * sw_piece.size()));
+    MGPU_RET(up(M.d_tb_piece, tb_piece.data(), sizeof(int) * tb_piece.size()));
+    MGPU_RET(up(M.d_pieces, pieces.data(), sizeof(TPieces) * pieces.size()));
+    MGPU_RET(up(M.d_poff, poff.data(), sizeof(int64_t) * poff.size()));
+    MGPU_RET(up(M.d_row0, row0.data(), sizeof(int) * nces));
+    if (!row_ces.empty()) MGPU_RET(up(M.d_row_ces, row_ces.data(), sizeof(int) * row_ces.size()));
+    if (az_chunks) {
+        k_chunk_order<<<M.nchunks, 256, 0, s>>>(M.d_az, M.d_c0, M.d_len, M.d_chunk_ces, M.d_chunk_lo, M.nsss,
+                                                M.d_order, M.d_abin);
+        MGPU_LAUNCHED();
+    }
     MGPU_HIP(hipEventRecord(pb.ev0, s));
     // kernels B_b: every entry summed by one thread in sample order
     if (M.nB > 0) MGPU_HIP(hipMemsetAsync(M.d_B, 0, sizeof(double) * M.nB, s));
@@ -756,6 +1025,22 @@ int templates_build(Problem &pb, const mgpu_templates *t) {
         MGPU_RET(pb.arena.alloc(&d_info, (size_t) nces));
         MGPU_RET(pb.arena.alloc(&d_rep, (size_t) nb));
         MGPU_RET(pb.arena.alloc(&d_sc, (size_t) nb));
+        // each block's factor and each CES's representative block, for the products with B^+
+        std::vector<int> ces_rep((size_t) nces);
+        std::vector<double> factor((size_t) nb);
+        for (int c = 0; c < nces; c++) {
+            int r = c * ndet;
+            for (int j = 0; j < ndet; j++)
+                if (w[(size_t) c * ndet + j] != 0.0) {
+                    r = c * ndet + j;
+                    break;
+                }
+            ces_rep[c] = r;
+            for (int b = c * ndet; b < (c + 1) * ndet; b++)
+                factor[b] = (w[b] != 0.0 && w[r] != 0.0) ? w[r] / w[b] : 0.0;
+        }
+        MGPU_RET(up(M.d_rep_blk, ces_rep.data(), sizeof(int) * nces));
+        MGPU_RET(up(M.d_scale, factor.data(), sizeof(double) * nb));
         for (int c = 0; c < nces;) {
             const int b0 = c * ndet;
             const int n = M.h_nt[b0];
@@ -775,18 +1060,11 @@ int templates_build(Problem &pb, const mgpu_templates *t) {
             std::vector<int> rep_blk((size_t) nrep), rep_of((size_t) nblk);
             std::vector<double> sc((size_t) nblk);
             for (int k = 0; k < nrep; k++) {
-                const int cb = (c_first + k) * ndet;
-                int r = cb;
-                for (int j2 = 0; j2 < ndet; j2++)
-                    if (w[(size_t) cb + j2] != 0.0) {
-                        r = cb + j2;
-                        break;
-                    }
+                const int cb = (c_first + k) * ndet, r = ces_rep[c_first + k];
                 rep_blk[k] = r;
-                for (int j2 = 0; j2 < ndet; j2++) {
-                    const int b = cb + j2;
+                for (int b = cb; b < cb + ndet; b++) {
                     rep_of[(size_t) (b - b0)] = k;
-                    sc[(size_t) (b - b0)] = (w[b] != 0.0 && w[r] != 0.0) ? w[r] / w[b] : 0.0;
+                    sc[(size_t) (b - b0)] = factor[b];
                 }
                 MGPU_HIP(hipMemcpyAsync(V + k * nn, M.d_B + M.h_boff[r], sizeof(double) * nn, hipMemcpyDeviceToDevice,
                                         s));
@@ -830,13 +1108,41 @@ int templates_build(Problem &pb, const mgpu_templates *t) {
 // ---------------------------------------------------------------------------
 // application
 // ---------------------------------------------------------------------------
+// kernels for at most 1, 4 or 16 Legendre orders and 2, 4 or 16 HWP slots
+#define MGPU_CLASSES(M, F)                              \
+    do {                                                \
+        const int p_ = (M).npoly, h_ = 2 * (M).nhwp;    \
+        if (p_ <= 1 && h_ <= 2) F(1, 2);                \
+        else if (p_ <= 1 && h_ <= 4) F(1, 4);           \
+        else if (p_ <= 1) F(1, 16);                     \
+        else if (p_ <= 4 && h_ <= 2) F(4, 2);           \
+        else if (p_ <= 4 && h_ <= 4) F(4, 4);           \
+        else if (p_ <= 4) F(4, 16);                     \
+        else if (h_ <= 4) F(16, 4);                     \
+        else F(16, 16);                                 \
+    } while (0)
+
 static int launch_tr(Problem &pb, const double *d_y, const double *scale, double *d_out) {
     Templates &M = pb.tm;
-    if (M.nitems == 0) return MGPU_OK;
-    k_tmpl_tr<<<(unsigned) M.nitems, kTW, 0, pb.stream>>>(M.d_items, d_y, scale, pb.tp.d_start, M.d_c0, M.ndet,
-                                                          M.d_perm, M.d_leg, M.d_hc, M.ncs, M.npoly, 2 * M.nhwp,
-                                                          M.d_off, d_out, pb.live_state);
+    if (M.ntot == 0) return MGPU_OK;
+    hipStream_t s = pb.stream;
+    const int az_here = M.d_order ? 1 : 0;
+    const TrArgs a{d_y, scale, pb.tp.d_start, M.d_c0, M.d_poff, M.d_len, M.d_chunk_ces, M.d_chunk_lo, M.d_chunk_p,
+                   M.d_chunk_h, M.d_ppiece, M.d_hpiece, M.d_pieces, M.d_order, M.d_abin, M.d_leg, M.d_hc, M.ncs,
+                   M.ndet, M.nchunks, M.npoly, 2 * M.nhwp, az_here ? M.nsss : 0, M.d_part, pb.live_state};
+#define MGPU_PART(NP, NH) k_tmpl_part<NP, NH><<<(unsigned) (M.nchunks * M.ndet), 256, 0, s>>>(a)
+    MGPU_CLASSES(M, MGPU_PART);
+#undef MGPU_PART
     MGPU_LAUNCHED();
+    k_tmpl_fin<<<grid_for(M.ntot * 16, 256), 256, 0, s>>>(M.d_part, M.d_poff, M.d_pieces, M.d_sw_piece, M.d_tb_piece,
+                                                          M.d_ns, M.d_nh, M.d_row_block, M.d_off, M.ntot, M.ndet,
+                                                          M.npoly, 2 * M.nhwp, M.nsss, az_here, d_out, pb.live_state);
+    MGPU_LAUNCHED();
+    if (M.nitems) {
+        k_tmpl_az<<<(unsigned) M.nitems, kTW, 0, s>>>(M.d_items, d_y, scale, pb.tp.d_start, M.d_c0, M.ndet, M.d_perm,
+                                                      M.d_off, d_out, pb.live_state);
+        MGPU_LAUNCHED();
+    }
     return MGPU_OK;
 }
 
@@ -864,20 +1170,21 @@ static int apply_tm(Problem &pb, const double *d_q, const double *in_scale, doub
     pb.prof.begin(MGPU_KT_TMPL, s);
     MGPU_RET(launch_tr(pb, d_q, in_scale, M.d_a1));
     if (M.ntot > 0) {  // (with no template class k_tmpl_sub reads no amplitude)
-        k_tmpl_binv<<<grid_for(M.ntot, 4), 256, 0, s>>>(M.d_Binv, M.d_boff, M.d_off, M.d_row_block, M.ntot, M.d_a1,
-                                                        M.d_a2, pb.live_state);
+        k_tmpl_binv<<<grid_for(M.nrows, 4), 256, 0, s>>>(M.d_Binv, M.d_boff, M.d_off, M.d_rep_blk, M.d_row_ces,
+                                                         M.d_row0, M.nrows, M.ndet, M.d_scale, M.d_a1, M.d_a2,
+                                                         pb.live_state);
         MGPU_LAUNCHED();
     }
-    if (d_q == d_y)
-        k_tmpl_sub<true><<<M.nwg_samples, 256, 0, s>>>(nullptr, in_scale, d_y, pb.tp.d_start, pb.tp.d_T0, M.ndet,
-                                                       M.d_c0, M.d_ns, M.d_nh, M.d_sweep, M.d_az, M.d_leg, M.d_hc,
-                                                       M.ncs, M.npoly, M.ground, M.nsss, 2 * M.nhwp, M.fsdt, M.d_off,
-                                                       M.d_a2, M.d_ces_of, M.d_len, pb.live_state);
-    else
-        k_tmpl_sub<false><<<M.nwg_samples, 256, 0, s>>>(d_q, in_scale, d_y, pb.tp.d_start, pb.tp.d_T0, M.ndet,
-                                                        M.d_c0, M.d_ns, M.d_nh, M.d_sweep, M.d_az, M.d_leg, M.d_hc,
-                                                        M.ncs, M.npoly, M.ground, M.nsss, 2 * M.nhwp, M.fsdt,
-                                                        M.d_off, M.d_a2, M.d_ces_of, M.d_len, pb.live_state);
+#define MGPU_SUB(NP, NH)                                                                                              \
+    do {                                                                                                              \
+        const auto k_ = d_q == d_y ? k_tmpl_sub<true, NP, NH> : k_tmpl_sub<false, NP, NH>;                            \
+        k_<<<M.nwg_samples, 256, 0, s>>>(d_q == d_y ? nullptr : d_q, in_scale, d_y, pb.tp.d_start, pb.tp.d_T0, M.ndet, \
+                                         M.d_c0, M.d_ns, M.d_nh, M.d_sweep, M.d_az, M.d_leg, M.d_hc, M.ncs, M.npoly,  \
+                                         M.ground, M.nsss, 2 * M.nhwp, M.fsdt, M.d_off, M.d_a2, M.d_ces_of, M.d_len,  \
+                                         pb.live_state);                                                              \
+    } while (0)
+    MGPU_CLASSES(M, MGPU_SUB);
+#undef MGPU_SUB
     MGPU_LAUNCHED();
     pb.prof.end(s);
     return MGPU_OK;
