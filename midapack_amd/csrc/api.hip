@@ -538,8 +538,8 @@ int mappraiser_gpu_pcg(mgpu_problem *h, const double *signal, const double *nois
     MGPU_ARG(pb.pc.built, "pcg before precond_build");
     if (!pb.d_sig) MGPU_RET(pb.arena.alloc(&pb.d_sig, (size_t) pb.pt.m));
     if (!pb.d_noise) MGPU_RET(pb.arena.alloc(&pb.d_noise, (size_t) pb.pt.m));
-    MGPU_HIP(hipMemcpyAsync(pb.d_sig, signal, sizeof(double) * pb.pt.m, hipMemcpyHostToDevice, pb.stream));
-    MGPU_HIP(hipMemcpyAsync(pb.d_noise, noise, sizeof(double) * pb.pt.m, hipMemcpyHostToDevice, pb.stream));
+    MGPU_RET(h2d_staged(pb.device, pb.d_sig, signal, sizeof(double) * pb.pt.m, pb.stream));
+    MGPU_RET(h2d_staged(pb.device, pb.d_noise, noise, sizeof(double) * pb.pt.m, pb.stream));
     mgpu_report r{};
     MGPU_RET(pcg_run(pb, pb.d_sig, pb.d_noise, tol, maxiter, stop_after, x, res_hist, &r));
     if (rep) *rep = r;

@@ -23,8 +23,14 @@ namespace mgpu {
 
 namespace {
 
-constexpr size_t kStageChunk = (size_t) 12 << 20;  // bytes per chunk (a multiple of 8, 12 and 16)
-constexpr size_t kStageMin = (size_t) 48 << 20;    // smaller copies go through hipMemcpyAsync
+constexpr size_t kStageChunk = (size_t) 12 << 20;  // bytes per chunk at most (a whole number of units)
+constexpr size_t kStageUnit = 48 << 10;            // chunks are multiples of it, and so of 8, 12 and 16
+// Plain copies below kStageMin go through hipMemcpyAsync; copies with host work
+// on every chunk (packing, side effects) are shared by a thread per kStageWork
+// bytes, two chunks each.  (A drop-in solve of 3.1 M samples, whose 38 MB of local
+// indices and side effects one thread took through a plain copy: 27 -> 11 ms.)
+constexpr size_t kStageMin = (size_t) 4 << 20;
+constexpr size_t kStageWork = (size_t) 256 << 10;
 constexpr int kMaxWorkers = 8;
 constexpr int kMaxDevices = 16;
 
@@ -40,6 +46,18 @@ struct StagePool {
 };
 
 StagePool g_pool;
+
+// workers and chunk size of a transfer
+struct StageSplit {
+    int workers;
+    size_t chunk, n;
+    StageSplit(size_t bytes, int most) {
+        workers = (int) std::min<size_t>((size_t) most, std::max<size_t>(1, bytes / kStageWork));
+        const size_t share = bytes / (2 * (size_t) workers) + 1;
+        chunk = std::min(kStageChunk, (share + kStageUnit - 1) / kStageUnit * kStageUnit);
+        n = (bytes + chunk - 1) / chunk;
+    }
+};
 
 unsigned char *buffer(int w, int b) { return g_pool.pinned + ((size_t) w * 2 + b) * kStageChunk; }
 
@@ -104,8 +122,9 @@ int h2d_staged(int device, void *d, const void *h, size_t bytes, hipStream_t s) 
     }
     std::lock_guard<std::mutex> lk(g_pool.busy);
     MGPU_RET(pool_ready(device));
-    const int W = g_pool.workers;
-    const size_t nch = (bytes + kStageChunk - 1) / kStageChunk;
+    const StageSplit sp(bytes, g_pool.workers);
+    const int W = sp.workers;
+    const size_t nch = sp.n;
     unsigned char *dd = (unsigned char *) d;
     const unsigned char *hh = (const unsigned char *) h;
     MGPU_RET(run_workers(device, W, [&](int w) -> int {
@@ -113,7 +132,7 @@ int h2d_staged(int device, void *d, const void *h, size_t bytes, hipStream_t s) 
         int j = 0;
         for (size_t k = (size_t) w; k < nch; k += (size_t) W, j++) {
             const int b = j & 1;
-            const size_t off = k * kStageChunk, len = std::min(kStageChunk, bytes - off);
+            const size_t off = k * sp.chunk, len = std::min(sp.chunk, bytes - off);
             // the buffer's previous DMA (of this or an earlier transfer) has finished
             MGPU_HIP(hipEventSynchronize(g_pool.ev[device][w][b]));
             std::memcpy(buffer(w, b), hh + off, len);
@@ -131,15 +150,16 @@ int h2d_staged(int device, void *d, const void *h, size_t bytes, hipStream_t s) 
 int h2d_staged_fill(int device, void *d, size_t bytes, const StageProducer &fill) {
     std::lock_guard<std::mutex> lk(g_pool.busy);
     MGPU_RET(pool_ready(device));
-    const int W = g_pool.workers;
-    const size_t nch = (bytes + kStageChunk - 1) / kStageChunk;
+    const StageSplit sp(bytes, g_pool.workers);
+    const int W = sp.workers;
+    const size_t nch = sp.n;
     unsigned char *dd = (unsigned char *) d;
     MGPU_RET(run_workers(device, W, [&](int w) -> int {
         hipStream_t st = g_pool.ws[device][w];
         int j = 0;
         for (size_t k = (size_t) w; k < nch; k += (size_t) W, j++) {
             const int b = j & 1;
-            const size_t off = k * kStageChunk, len = std::min(kStageChunk, bytes - off);
+            const size_t off = k * sp.chunk, len = std::min(sp.chunk, bytes - off);
             MGPU_HIP(hipEventSynchronize(g_pool.ev[device][w][b]));
             fill(off, buffer(w, b), len);
             MGPU_HIP(hipMemcpyAsync(dd + off, buffer(w, b), len, hipMemcpyHostToDevice, st));
@@ -154,7 +174,7 @@ int h2d_staged_fill(int device, void *d, size_t bytes, const StageProducer &fill
 
 int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t after, const StageConsumer *consume) {
     std::unique_lock<std::mutex> lk(g_pool.busy, std::defer_lock);
-    if (bytes >= kStageMin) lk.try_lock();
+    if (bytes >= (consume ? kStageWork : kStageMin)) lk.try_lock();
     if (!lk.owns_lock()) {
         // small or pool busy: one copy, then the consumer over the whole array
         MGPU_HIP(hipEventSynchronize(after));
@@ -168,15 +188,16 @@ int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t afte
         return MGPU_OK;
     }
     MGPU_RET(pool_ready(device));
-    const int W = g_pool.workers;
-    const size_t nch = (bytes + kStageChunk - 1) / kStageChunk;
+    const StageSplit sp(bytes, g_pool.workers);
+    const int W = sp.workers;
+    const size_t nch = sp.n;
     const unsigned char *dd = (const unsigned char *) d;
     unsigned char *hh = (unsigned char *) h;
     MGPU_HIP(hipEventSynchronize(after));  // the pool's streams wait on no other stream
     return run_workers(device, W, [&](int w) -> int {
         hipStream_t st = g_pool.ws[device][w];
         auto issue = [&](size_t k, int b) -> int {
-            const size_t off = k * kStageChunk, len = std::min(kStageChunk, bytes - off);
+            const size_t off = k * sp.chunk, len = std::min(sp.chunk, bytes - off);
             MGPU_HIP(hipEventSynchronize(g_pool.ev[device][w][b]));
             MGPU_HIP(hipMemcpyAsync(buffer(w, b), dd + off, len, hipMemcpyDeviceToHost, st));
             MGPU_HIP(hipEventRecord(g_pool.ev[device][w][b], st));
@@ -189,7 +210,7 @@ int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t afte
             const int b = j & 1;
             if (k + W < nch) MGPU_RET(issue(k + W, b ^ 1));  // next chunk in flight meanwhile
             MGPU_HIP(hipEventSynchronize(g_pool.ev[device][w][b]));
-            const size_t off = k * kStageChunk, len = std::min(kStageChunk, bytes - off);
+            const size_t off = k * sp.chunk, len = std::min(sp.chunk, bytes - off);
             if (consume)
                 (*consume)(off, buffer(w, b), len);
             else

@@ -111,17 +111,17 @@ bool serving_thread();
 // Copies between the caller's pageable host arrays and the device through a
 // process-wide pool of pinned staging buffers (hostio.hip).  h2d_staged: when
 // it returns, the host array may be reused, and work queued on s afterwards
-// sees the data (copies of 48 MiB and more are complete on return; smaller
+// sees the data (copies of 4 MiB and more are complete on return; smaller
 // ones are queued on s).  d2h_staged: the copies start once the event `after` has
 // completed; when it returns the data has been delivered, either copied to h or, with
 // a consumer, handed to consume(offset, chunk, bytes) chunk by chunk (called
-// from several threads at once on disjoint chunks; offsets are multiples of
-// 12 MiB).
+// from several threads at once on disjoint chunks; offsets and all chunks but the
+// last are multiples of 48 KiB).
 using StageConsumer = std::function<void(size_t off, const void *chunk, size_t bytes)>;
 // h2d_staged_fill: `bytes` of device data produced on the host chunk by chunk:
 // fill(off, chunk, len) writes bytes [off, off + len) of the data into the
 // pinned chunk (called from several threads at once on disjoint chunks;
-// offsets are multiples of 12 MiB).  Complete when the call returns.
+// offsets and all chunks but the last are multiples of 48 KiB).  Complete when the call returns.
 using StageProducer = std::function<void(size_t off, void *chunk, size_t bytes)>;
 int h2d_staged_fill(int device, void *d, size_t bytes, const StageProducer &fill);
 int h2d_staged(int device, void *d, const void *h, size_t bytes, hipStream_t s);

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as ct
 import os
+from concurrent.futures import ThreadPoolExecutor
 from dataclasses import dataclass
 
 import numpy as np
@@ -537,6 +538,29 @@ class GLSResult:
     signal: np.ndarray
 
 
+_COPY_CHUNK = 4 << 20  # bytes
+
+
+def _copies(*arrays):
+    """C-contiguous copies of the arrays.  Large ones are copied by several
+    threads (numpy releases the interpreter lock): most of a copy's time is the
+    first touch of its pages, which one thread does at a few GB/s."""
+    out = [np.empty(a.shape, a.dtype) for a in arrays]
+    parts = []
+    for d, a in zip(out, arrays):
+        n = max(1, _COPY_CHUNK // max(1, a.itemsize))
+        d, a = d.reshape(-1), a.reshape(-1)
+        parts += [(d[i:i + n], a[i:i + n]) for i in range(0, a.size, n)]
+    threads = min(8, os.cpu_count() or 1, len(parts) // 2)
+    if threads < 2:
+        for p in parts:
+            np.copyto(*p)
+    else:
+        with ThreadPoolExecutor(threads) as ex:
+            list(ex.map(lambda p: np.copyto(*p), parts))
+    return out
+
+
 def pcg_gls(pix, weights, signal, noise, block_sizes, lam, invtt, tol=1e-8, maxiter=500, nnz=3,
             opts: Options | None = None, outpath: str | None = None, ref: str | None = None,
             inplace: bool = False) -> GLSResult:
@@ -551,9 +575,7 @@ def pcg_gls(pix, weights, signal, noise, block_sizes, lam, invtt, tol=1e-8, maxi
                 raise GPUError("inplace=True needs writable C-contiguous int32 pix and float64 weights/signal")
         p, w, s = pix, weights, signal
     else:
-        p = _c(pix, np.int32).copy()
-        w = _c(weights, np.float64).copy()
-        s = _c(signal, np.float64).copy()
+        p, w, s = _copies(_c(pix, np.int32), _c(weights, np.float64), _c(signal, np.float64))
     nz = _c(noise, np.float64)
     m = p.size // nnz
     bs = _c(block_sizes, np.int32)
