@@ -298,6 +298,7 @@ struct Pointing {
     float2 *d_cw12f = nullptr;
     int *d_pixg = nullptr; // [npix0] global pixel number p (valid pixels, increasing)
     int *d_chunk_perm = nullptr; // [ceil(m/kChunk)] chunk processed by P's workgroup b
+    std::vector<int> h_chunk_key;   // smallest local pixel of every P chunk (INT32_MAX: none)
     std::vector<int> h_chunk_order; // the chunks in P's order before they are dealt to the XCDs
     int *d_perm_run = nullptr;   // chunks of the segments still running (segmented PCG)
     int nch_run = -1;            // their count (-1: every chunk, d_chunk_perm)
@@ -592,8 +593,9 @@ int pointing_make_fp32(Problem &pb);
 int pointing_compact(Problem &pb, const unsigned *d_kept);
 
 // y = P x (FP64); optional fused per-block partials when tp has blocks
-int launch_matvec(Problem &pb, const double *d_x, double *d_y, bool partials);
-int launch_matvec_f32(Problem &pb, const float *d_x, float *d_y, bool partials);
+// diag: lambda 1, the product weighted by T_b[0] (see diag_in_p)
+int launch_matvec(Problem &pb, const double *d_x, double *d_y, bool partials, bool diag = false);
+int launch_matvec_f32(Problem &pb, const float *d_x, float *d_y, bool partials, bool diag = false);
 // x = P^T y; optional fused partial dots of <x, hvec> into d_dot (one per workgroup)
 int launch_trmatvec(Problem &pb, const double *d_y, double *d_x, const double *d_hvec,
                     double *d_dotpart, int *nparts);
@@ -601,7 +603,6 @@ int launch_trmatvec_f32(Problem &pb, const float *d_y, double *d_x, const double
                         double *d_dotpart, int *nparts);
 int trmatvec_nparts(const Problem &pb);
 // smallest valid local pixel of every P chunk (INT32_MAX: none), on the host
-int pointing_chunk_keys(Problem &pb, std::vector<int> &key);
 
 // Block definitions and the Toeplitz set-up (defineBlocks_avg, tpltz_init).
 // invtt holds the band of every block, block b's band at the running sum of
@@ -613,6 +614,8 @@ int toeplitz_plan(Problem &pb, const int *block_sizes, int nb, int lambda, const
                   const double *h_invtt, const int *block_lambda = nullptr, const int *block_log2n = nullptr);
 // N^-1 on d_in (its per-block partials must already be in tp.d_partials unless
 // compute_partials) -> d_out (may not alias d_in)
+// N^-1 (s + n) with white noise in one pass
+int toeplitz_diag_sum(Problem &pb, const double *d_s, const double *d_n, double *d_out);
 int toeplitz_apply(Problem &pb, const double *d_in, double *d_out, bool compute_partials);
 int toeplitz_apply_f32(Problem &pb, const float *d_in, float *d_out, bool compute_partials);
 // scratch of one N^-1 product: partial sums [nchunks + nb], means [nb], slice

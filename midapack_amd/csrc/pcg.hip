@@ -522,8 +522,7 @@ int segments_ensure(Problem &pb) {
     MGPU_HIP(hipStreamSynchronize(s));
     // segment of every P chunk (by its smallest pixel) and Toeplitz block (by its
     // first chunk): batch items are padded to whole chunks, so neither straddles two
-    std::vector<int> key;
-    MGPU_RET(pointing_chunk_keys(pb, key));
+    const std::vector<int> &key = pb.pt.h_chunk_key;
     const int nch = (int) key.size();
     std::vector<int> cseg((size_t) nch, -1);
     for (int c = 0; c < nch; c++)
@@ -641,14 +640,21 @@ int ensure_work(Problem &pb) {
     return MGPU_OK;
 }
 
+// white noise: N^-1 is a weight per block, which P applies itself (not with the
+// block means of stbmmProd, nor with templates, whose kernels weight the samples)
+static bool diag_in_p(const Problem &pb) {
+    return pb.tp.lambda == 1 && !pb.tm.live && !(pb.stbmm_offsets && pb.tp.offset_mode != MGPU_OFFSET_NONE);
+}
+
 // A v = P^T N^-1 P v in FP64 (map -> map), fused <v, Av> partials optional
 int apply_A64(Problem &pb, const double *d_v, double *d_out, double *d_dot) {
+    const bool diag = diag_in_p(pb);
     pb.prof.begin(MGPU_KT_P, pb.stream);
-    MGPU_RET(launch_matvec(pb, d_v, pb.d_tod, true));
+    MGPU_RET(launch_matvec(pb, d_v, diag ? pb.d_tod2 : pb.d_tod, true, diag));
     pb.prof.end(pb.stream);
     if (pb.tm.live)  // apply_weights and the template part of PCG_GLS_templates (pcg_true.c:426-458)
         MGPU_RET(templates_noise(pb, pb.d_tod, pb.d_tod2));
-    else
+    else if (!diag)
         MGPU_RET(toeplitz_apply(pb, pb.d_tod, pb.d_tod2, false));
     pb.prof.begin(MGPU_KT_PT, pb.stream);
     MGPU_RET(launch_trmatvec(pb, pb.d_tod2, d_out, d_dot ? d_v : nullptr, d_dot, nullptr));
@@ -658,10 +664,11 @@ int apply_A64(Problem &pb, const double *d_v, double *d_out, double *d_dot) {
 
 // q = A v in FP32 products; pb.d_mapf holds v's FP32 copy (k_hupdate writes it)
 static int apply_A32(Problem &pb, const double *d_v, double *d_out, double *d_dot) {
+    const bool diag = diag_in_p(pb);
     pb.prof.begin(MGPU_KT_P, pb.stream);
-    MGPU_RET(launch_matvec_f32(pb, pb.d_mapf, pb.d_todf, true));
+    MGPU_RET(launch_matvec_f32(pb, pb.d_mapf, diag ? pb.d_tod2f : pb.d_todf, true, diag));
     pb.prof.end(pb.stream);
-    MGPU_RET(toeplitz_apply_f32(pb, pb.d_todf, pb.d_tod2f, false));
+    if (!diag) MGPU_RET(toeplitz_apply_f32(pb, pb.d_todf, pb.d_tod2f, false));
     pb.prof.begin(MGPU_KT_PT, pb.stream);
     MGPU_RET(launch_trmatvec_f32(pb, pb.d_tod2f, d_out, d_dot ? d_v : nullptr, d_dot, nullptr));
     pb.prof.end(pb.stream);
@@ -747,12 +754,16 @@ int pcg_run(Problem &pb, const double *d_signal, const double *d_noise, double t
         ~TemplatesLive() { pb.tm.live = false; }
     } tm_live{pb};
     pb.tm.live = pb.tm.on;
-    k_rhs_tod<<<grid_for(m, 256), 256, 0, s>>>(d_signal, d_noise, pb.d_tod, m);
-    MGPU_LAUNCHED();
-    if (pb.tm.live)  // pcg_true.c:318-371
-        MGPU_RET(templates_noise(pb, pb.d_tod, pb.d_tod2));
-    else
-        MGPU_RET(toeplitz_apply(pb, pb.d_tod, pb.d_tod2, true));
+    if (diag_in_p(pb)) {
+        MGPU_RET(toeplitz_diag_sum(pb, d_signal, d_noise, pb.d_tod2));
+    } else {
+        k_rhs_tod<<<grid_for(m, 256), 256, 0, s>>>(d_signal, d_noise, pb.d_tod, m);
+        MGPU_LAUNCHED();
+        if (pb.tm.live)  // pcg_true.c:318-371
+            MGPU_RET(templates_noise(pb, pb.d_tod, pb.d_tod2));
+        else
+            MGPU_RET(toeplitz_apply(pb, pb.d_tod, pb.d_tod2, true));
+    }
     MGPU_RET(launch_trmatvec(pb, pb.d_tod2, gA, nullptr, nullptr, nullptr));
     MGPU_HIP(hipMemcpyAsync(bvec, gA, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     if (two) {

@@ -46,8 +46,11 @@ constexpr int kClassifyGrid = 2048; // grid-stride validation: 8 workgroups per 
 // status bits: 1 = malformed row, 2 = trash row present, 4 = I weight != 1.
 // Grid-stride over the samples, one reduction per workgroup: the three
 // device-wide atomics are issued once per workgroup instead of once per wave.
+// The (Q, U) weights are copied to P's w12 in the same pass over the weights (64 x
+// 2^20 samples: 741 us, and 280 us for k_assign, which read them again: 526 + 638).
 __global__ __launch_bounds__(256) void k_classify(const int *__restrict__ pix, const double *__restrict__ w,
-                                                  int64_t m, int *__restrict__ p_of_t, int *__restrict__ status,
+                                                  int64_t m, int *__restrict__ p_of_t,
+                                                  double2 *__restrict__ w12, int *__restrict__ status,
                                                   int *__restrict__ pmin, int *__restrict__ pmax,
                                                   int *__restrict__ first_bad) {
     __shared__ int slo[4], shi[4], sst[4];
@@ -73,6 +76,7 @@ __global__ __launch_bounds__(256) void k_classify(const int *__restrict__ pix, c
             atomicMin(first_bad, (int) t);  // m < 2^31
         }
         if (w[3 * t] != 1.0) st |= 4;
+        w12[t] = make_double2(w[3 * t + 1], w[3 * t + 2]);
         p_of_t[t] = p;
         if (p >= 0) {
             lo = min(lo, p);
@@ -113,19 +117,16 @@ __global__ void k_mark(const int *__restrict__ p_of_t, int64_t m, int pmin, unsi
     }
 }
 
-// w: the caller's weights (3 per sample), or nullptr when the Q/U weights were
-// uploaded packed (they are then P's w12 already and w12 is not written)
+// w: the caller's weights (3 per sample), read where the I weights are not all 1 (w0)
 __global__ void k_assign(const int *__restrict__ p_of_t, int64_t m, int pmin, const unsigned *__restrict__ rank,
                          const double *__restrict__ w, int *__restrict__ q, double *__restrict__ w0,
-                         double2 *__restrict__ w12, unsigned *__restrict__ key, int *__restrict__ tval,
-                         unsigned trash_key) {
+                         unsigned *__restrict__ key, int *__restrict__ tval, unsigned trash_key) {
     int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (t < m) {
         int p = p_of_t[t];
         int qq = p >= 0 ? (int) rank[p - pmin] : -1;
         q[t] = qq;
         if (w0) w0[t] = w[3 * t];
-        if (w) w12[t] = make_double2(w[3 * t + 1], w[3 * t + 2]);
         key[t] = qq >= 0 ? (unsigned) qq : trash_key;
         tval[t] = (int) t;
     }
@@ -174,18 +175,29 @@ __global__ void k_fill_ell(const int *__restrict__ off, const int *__restrict__ 
         lo = off[qq];
         hi = off[qq + 1];
     }
-    for (int64_t i = 0; i < width; i++) {
-        int64_t dst = b0 + i * kSlice + lane;
-        int h = lo + (int) i;
-        if (h < hi) {
-            int t = st[h];
-            ct[dst] = t;
-            if (W0) cw0[dst] = w0[t];
-            cw12[dst] = w12[t];
-        } else {
-            ct[dst] = -1;
-            if (W0) cw0[dst] = 0.0;
-            cw12[dst] = make_double2(0.0, 0.0);
+    // hits whose (dependent) loads are in flight together (64 x 2^20 samples: one 1530 us, eight 664 us)
+    constexpr int U = 8;
+    for (int64_t i0 = 0; i0 < width; i0 += U) {
+        int t[U];
+        double2 wv[U];
+        double w0v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int h = lo + (int) i0 + u;
+            t[u] = h < hi ? st[h] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            wv[u] = t[u] >= 0 ? w12[t[u]] : make_double2(0.0, 0.0);
+            if (W0) w0v[u] = t[u] >= 0 ? w0[t[u]] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (i0 + u >= width) break;
+            const int64_t dst = b0 + (i0 + u) * kSlice + lane;
+            ct[dst] = t[u];
+            if (W0) cw0[dst] = w0v[u];
+            cw12[dst] = wv[u];
         }
     }
 }
@@ -294,7 +306,7 @@ __global__ __launch_bounds__(256) void k_chunk_key(const int *__restrict__ q, in
     if (threadIdx.x == 0) key[blockIdx.x] = min(min(red[0], red[1]), min(red[2], red[3]));
 }
 
-int pointing_chunk_keys(Problem &pb, std::vector<int> &key) {
+static int chunk_keys(Problem &pb, std::vector<int> &key) {
     Pointing &P = pb.pt;
     hipStream_t s = pb.stream;
     const int nch = (int) ((P.m + kChunk - 1) / kChunk);
@@ -313,8 +325,9 @@ static int build_chunk_order(Problem &pb) {
     Pointing &P = pb.pt;
     hipStream_t s = pb.stream;
     const int nch = (int) ((P.m + kChunk - 1) / kChunk);
-    std::vector<int> key, order((size_t) nch), perm((size_t) nch);
-    MGPU_RET(pointing_chunk_keys(pb, key));
+    std::vector<int> order((size_t) nch), perm((size_t) nch);
+    MGPU_RET(chunk_keys(pb, P.h_chunk_key));
+    const std::vector<int> &key = P.h_chunk_key;
     // Groups of kChunkGroup consecutive chunks, sorted by their smallest pixel:
     // the map rows a group gathers stay in L2 while the detectors' passes over
     // them run back to back, and each group streams its pointing from HBM as
@@ -402,7 +415,9 @@ int pointing_build(Problem &pb, const int *d_pix, const double *d_wts, int64_t m
     int init[4] = {0, INT32_MAX, INT32_MIN, INT32_MAX};
     MGPU_HIP(hipMemcpyAsync(d_stat, init, sizeof(init), hipMemcpyHostToDevice, s));
     const unsigned gcl = (unsigned) std::min<int64_t>(kClassifyGrid, (m + 255) / 256);
-    k_classify<<<gcl, 256, 0, s>>>(d_pix, d_wts, m, d_p, d_stat, d_stat + 1, d_stat + 2, d_stat + 3);
+    double2 *d_w12;
+    MGPU_RET(pb.arena.alloc(&d_w12, (size_t) m));
+    k_classify<<<gcl, 256, 0, s>>>(d_pix, d_wts, m, d_p, d_w12, d_stat, d_stat + 1, d_stat + 2, d_stat + 3);
     MGPU_LAUNCHED();
     int hst[4];
     MGPU_HIP(hipMemcpyAsync(hst, d_stat, sizeof(hst), hipMemcpyDeviceToHost, s));
@@ -417,7 +432,7 @@ int pointing_build(Problem &pb, const int *d_pix, const double *d_wts, int64_t m
     }
     MGPU_ARG(hst[1] != INT32_MAX, "no valid sample: every sample is flagged");
     P.unit_w0 = !(hst[0] & 4);
-    MGPU_RET(pointing_build_from_p(pb, d_p, hst[1], hst[2], (hst[0] & 2) != 0, d_wts, nullptr));
+    MGPU_RET(pointing_build_from_p(pb, d_p, hst[1], hst[2], (hst[0] & 2) != 0, d_wts, d_w12));
     pb.arena.release(d_p);
     return MGPU_OK;
 }
@@ -434,8 +449,9 @@ int pointing_build_packed(Problem &pb, const int *d_p, double2 *d_w12, int64_t m
 }
 
 // the pointing tables from each sample's global pixel p (-1: flagged): local
-// pixel ids, Q/U weights (from the caller's weights d_wts, or adopted from the
-// packed upload d_w12), the sample order by pixel and the sliced ELL of P^T
+// pixel ids, Q/U weights (d_w12, adopted), I weights (from the caller's weights
+// d_wts, not read when they are all 1), the sample order by pixel and the sliced
+// ELL of P^T
 int pointing_build_from_p(Problem &pb, const int *d_p, int pmin, int pmax, bool any_flagged, const double *d_wts,
                           double2 *d_w12) {
     Pointing &P = pb.pt;
@@ -461,10 +477,7 @@ int pointing_build_from_p(Problem &pb, const int *d_p, int pmin, int pmax, bool 
 
     MGPU_RET(pb.arena.alloc(&P.d_q, (size_t) m));
     if (!P.unit_w0) MGPU_RET(pb.arena.alloc(&P.d_w0, (size_t) m));
-    if (d_w12)
-        P.d_w12 = d_w12;  // the packed upload is P's Q/U weights (sample order)
-    else
-        MGPU_RET(pb.arena.alloc(&P.d_w12, (size_t) m));
+    P.d_w12 = d_w12;
     MGPU_RET(pb.arena.alloc(&P.d_pixg, (size_t) P.npix0));
     unsigned *d_key, *d_skey;
     int *d_t;
@@ -472,7 +485,7 @@ int pointing_build_from_p(Problem &pb, const int *d_p, int pmin, int pmax, bool 
     MGPU_RET(pb.arena.alloc(&d_skey, (size_t) m));
     MGPU_RET(pb.arena.alloc(&d_t, (size_t) m));
     MGPU_RET(pb.arena.alloc(&P.d_cst, (size_t) m));
-    k_assign<<<grid_for(m, 256), 256, 0, s>>>(d_p, m, pmin, d_rank, d_wts, P.d_q, P.d_w0, P.d_w12, d_key, d_t,
+    k_assign<<<grid_for(m, 256), 256, 0, s>>>(d_p, m, pmin, d_rank, d_wts, P.d_q, P.d_w0, d_key, d_t,
                                               (unsigned) P.npix0);
     MGPU_LAUNCHED();
     k_pixg<<<grid_for(span, 256), 256, 0, s>>>(d_flags, d_rank, span, pmin, P.d_pixg);
@@ -625,14 +638,16 @@ __device__ __forceinline__ double wg_sum_256(double v, double *red) {
 // streaming load of its chunks is issued before the map gathers.  (Two chunks
 // per workgroup in FP32, for more bytes in flight per lane, measured slower on
 // the 64 x 2^20 raster: 0.248 against 0.232 ms per launch.)
-template <typename TX, typename TW, typename TW2, bool W0, bool PARTIALS, int CPW>
+// DIAG (white noise): y = T_b[0] (P x), the weighting of apply_weights in the same
+// pass, with k_diag's products (24 x 500009 samples: a pass of 40 us less an iteration).
+template <typename TX, typename TW, typename TW2, bool W0, bool PARTIALS, bool DIAG, int CPW>
 __global__ __launch_bounds__(kPBlock) void k_matvec(const int *__restrict__ q, const TW *__restrict__ w0,
                                                     const TW2 *__restrict__ w12, const TX *__restrict__ x,
                                                     TX *__restrict__ y, int64_t m, const int64_t *__restrict__ start,
                                                     const int *__restrict__ chunk_block, int nb,
                                                     double *__restrict__ partials, const int *__restrict__ perm,
                                                     int nperm, const int *__restrict__ chunk_seg,
-                                                    const int *__restrict__ state) {
+                                                    const int *__restrict__ state, const double *__restrict__ T0) {
     __shared__ double red[kPBlock / 64];
     constexpr int PER = kChunk / kPBlock;
     int64_t cs[CPW];
@@ -676,6 +691,13 @@ __global__ __launch_bounds__(kPBlock) void k_matvec(const int *__restrict__ q, c
                 acc += (TX) wv[j][i].y * x2;
                 v = acc;
             }
+            if constexpr (DIAG) {
+                if (live[j]) {  // the block of a lane's sample: the chunk's first, or one of the next
+                    int b = chunk_block[cs[j]];
+                    while (b < nb && t >= start[b + 1]) b++;
+                    if (b < nb) v = (TX) T0[b] * v;
+                }
+            }
             if (live[j] && t < m) y[t] = v;
             yv[j][i] = v;
         }
@@ -702,16 +724,14 @@ __global__ __launch_bounds__(kPBlock) void k_matvec(const int *__restrict__ q, c
 }
 
 template <typename TX, typename TW, typename TW2>
-static int launch_matvec_t(Problem &pb, const TX *d_x, TX *d_y, bool partials, const TW *w0, const TW2 *w12) {
+static int launch_matvec_t(Problem &pb, const TX *d_x, TX *d_y, bool partials, bool diag, const TW *w0,
+                           const TW2 *w12) {
     constexpr int CPW = 1;  // chunks per workgroup (both precisions)
     const Pointing &P = pb.pt;
     const ToeplitzPlan &T = pb.tp;
     int nperm = (int) grid_for(P.m, kChunk);
     partials = partials && T.nb > 0 && T.d_partials && T.d_chunk_block && T.lambda > 1 &&
                T.offset_mode != MGPU_OFFSET_NONE;
-    const int *q = P.d_q;
-    const int64_t *st = T.d_start;
-    const int *cb = T.d_chunk_block;
     const int *pm = P.d_chunk_perm;
     MGPU_ARG(pm, "pointing has no chunk order");
     if (pb.live_state && P.nch_run >= 0) {  // segmented PCG: the running segments' chunks only
@@ -721,31 +741,38 @@ static int launch_matvec_t(Problem &pb, const TX *d_x, TX *d_y, bool partials, c
     }
     const unsigned g = (unsigned) ((nperm + CPW - 1) / CPW);
     const int *cs = pb.sg.d_chunk_seg, *ls = cs ? pb.live_state : nullptr;
+    auto launch = [&](auto kern) {
+        kern<<<g, kPBlock, 0, pb.stream>>>(P.d_q, P.unit_w0 ? nullptr : w0, w12, d_x, d_y, P.m, T.d_start,
+                                           T.d_chunk_block, T.nb, partials ? T.d_partials : nullptr, pm, nperm, cs, ls,
+                                           T.d_T0);
+    };
+#define MGPU_P(W0, PART, DIAG) launch(k_matvec<TX, TW, TW2, W0, PART, DIAG, CPW>)
     if (P.unit_w0) {
-        if (partials)
-            k_matvec<TX, TW, TW2, false, true, CPW><<<g, kPBlock, 0, pb.stream>>>(
-                    q, nullptr, w12, d_x, d_y, P.m, st, cb, T.nb, T.d_partials, pm, nperm, cs, ls);
+        if (diag)
+            MGPU_P(false, false, true);
+        else if (partials)
+            MGPU_P(false, true, false);
         else
-            k_matvec<TX, TW, TW2, false, false, CPW><<<g, kPBlock, 0, pb.stream>>>(
-                    q, nullptr, w12, d_x, d_y, P.m, st, cb, T.nb, nullptr, pm, nperm, cs, ls);
+            MGPU_P(false, false, false);
     } else {
-        if (partials)
-            k_matvec<TX, TW, TW2, true, true, CPW><<<g, kPBlock, 0, pb.stream>>>(
-                    q, w0, w12, d_x, d_y, P.m, st, cb, T.nb, T.d_partials, pm, nperm, cs, ls);
+        if (diag)
+            MGPU_P(true, false, true);
+        else if (partials)
+            MGPU_P(true, true, false);
         else
-            k_matvec<TX, TW, TW2, true, false, CPW><<<g, kPBlock, 0, pb.stream>>>(
-                    q, w0, w12, d_x, d_y, P.m, st, cb, T.nb, nullptr, pm, nperm, cs, ls);
+            MGPU_P(true, false, false);
     }
+#undef MGPU_P
     MGPU_LAUNCHED();
     return MGPU_OK;
 }
 
-int launch_matvec(Problem &pb, const double *d_x, double *d_y, bool partials) {
-    return launch_matvec_t<double, double, double2>(pb, d_x, d_y, partials, pb.pt.d_w0, pb.pt.d_w12);
+int launch_matvec(Problem &pb, const double *d_x, double *d_y, bool partials, bool diag) {
+    return launch_matvec_t<double, double, double2>(pb, d_x, d_y, partials, diag, pb.pt.d_w0, pb.pt.d_w12);
 }
 
-int launch_matvec_f32(Problem &pb, const float *d_x, float *d_y, bool partials) {
-    return launch_matvec_t<float, float, float2>(pb, d_x, d_y, partials, pb.pt.d_w0f, pb.pt.d_w12f);
+int launch_matvec_f32(Problem &pb, const float *d_x, float *d_y, bool partials, bool diag) {
+    return launch_matvec_t<float, float, float2>(pb, d_x, d_y, partials, diag, pb.pt.d_w0f, pb.pt.d_w12f);
 }
 
 // ---------------------------------------------------------------------------

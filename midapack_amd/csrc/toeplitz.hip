@@ -1048,14 +1048,16 @@ __device__ __forceinline__ int wg_block_of(const int64_t *__restrict__ start, in
     return b;
 }
 
+// (n: the input is y + n, the right-hand side's timestream)
 template <typename R>
-__global__ __launch_bounds__(256) void k_diag(const R *__restrict__ y, R *__restrict__ z, int64_t m,
-                                              const int64_t *__restrict__ start, int nb,
+__global__ __launch_bounds__(256) void k_diag(const R *__restrict__ y, const R *__restrict__ n, R *__restrict__ z,
+                                              int64_t m, const int64_t *__restrict__ start, int nb,
                                               const double *__restrict__ T0) {
     int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= m) return;
     const int b = wg_block_of(start, nb, t);
-    z[t] = b < nb ? (R) T0[b] * y[t] : y[t];
+    const R v = n ? (y[t] + n[t]) - (R) 0 : y[t];
+    z[t] = b < nb ? (R) T0[b] * v : v;
 }
 
 // lambda == 1 with stbmmProd's offsets (toeplitz_wizard.c:86-95 ahead of the
@@ -1845,7 +1847,7 @@ static int toeplitz_apply_t(Problem &pb, const R *d_in, R *d_out, bool compute_p
             MGPU_LAUNCHED();
             k_diag_mean<R><<<grid_for(T.m, 256), 256, 0, s>>>(d_in, d_out, T.m, T.d_start, T.nb, T.d_T0, sc.mean);
         } else {
-            k_diag<R><<<grid_for(T.m, 256), 256, 0, s>>>(d_in, d_out, T.m, T.d_start, T.nb, T.d_T0);
+            k_diag<R><<<grid_for(T.m, 256), 256, 0, s>>>(d_in, nullptr, d_out, T.m, T.d_start, T.nb, T.d_T0);
         }
         MGPU_LAUNCHED();
         return MGPU_OK;
@@ -1891,6 +1893,13 @@ static int toeplitz_apply_t(Problem &pb, const R *d_in, R *d_out, bool compute_p
 }
 
 static ToeplitzScratch plan_scratch(const ToeplitzPlan &T) { return {T.d_partials, T.d_mean, T.d_edge_part}; }
+
+int toeplitz_diag_sum(Problem &pb, const double *d_s, const double *d_n, double *d_out) {
+    const ToeplitzPlan &T = pb.tp;
+    k_diag<double><<<grid_for(T.m, 256), 256, 0, pb.stream>>>(d_s, d_n, d_out, T.m, T.d_start, T.nb, T.d_T0);
+    MGPU_LAUNCHED();
+    return MGPU_OK;
+}
 
 int toeplitz_apply(Problem &pb, const double *d_in, double *d_out, bool compute_partials) {
     return toeplitz_apply_t<double>(pb, d_in, d_out, compute_partials, plan_scratch(pb.tp));
