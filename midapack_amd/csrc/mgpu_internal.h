@@ -238,6 +238,7 @@ struct ToeplitzPlan {
     int nb = 0;
     int64_t m = 0;
     int64_t covered = 0;             // sum of block sizes (samples past it are left unchanged)
+    int64_t max_block = 0;           // samples of the longest block
     std::vector<int64_t> h_start;    // nb+1 block starts
     int64_t *d_start = nullptr;      // nb+1
     double *d_T0 = nullptr;          // nb, T_b[0]

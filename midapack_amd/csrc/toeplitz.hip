@@ -405,6 +405,39 @@ __device__ __forceinline__ double mean_out_of(const double *__restrict__ edge_pa
     return s / (double) n;
 }
 
+// Mean of a block from its chunks' partial sums: kMeanSums sums a lane, of every
+// 64 * kMeanSums-th partial, added in a fixed order.  One wave can hold all of them
+// (wave_block_mean: eight loads in flight) or one wave each (k_wave_mean, for long
+// blocks): the same bits.
+constexpr int kMeanSums = 8;
+struct MeanArgs {
+    const double *partials;  // nullptr: the means are not computed here
+    const int64_t *start;
+};
+// the lanes' sums added up, over the block's length; every lane gets it, in scalar registers
+__device__ __forceinline__ double mean_of_sums(double (&acc)[kMeanSums], int64_t n) {
+#pragma unroll
+    for (int h = kMeanSums / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (int k = 0; k < h; k++) acc[k] += acc[k + h];
+    double s = acc[0];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    const unsigned long long w = (unsigned long long) __double_as_longlong(s);
+    const unsigned w0 = (unsigned) __builtin_amdgcn_readfirstlane((int) (unsigned) w);
+    const unsigned w1 = (unsigned) __builtin_amdgcn_readfirstlane((int) (unsigned) (w >> 32));
+    return __longlong_as_double((long long) (((unsigned long long) w1 << 32) | w0)) / (double) n;
+}
+__device__ __forceinline__ double wave_block_mean(const MeanArgs &a, int b) {
+    const int64_t lo = a.start[b], hi = a.start[b + 1];
+    const int64_t last = (hi - 1) / kChunk;
+    double acc[kMeanSums] = {};
+    for (int64_t c0 = lo / kChunk + (threadIdx.x & 63); c0 <= last; c0 += 64 * kMeanSums)
+#pragma unroll
+        for (int k = 0; k < kMeanSums; k++)
+            if (c0 + 64 * k <= last) acc[k] += a.partials[c0 + 64 * k + b];
+    return mean_of_sums(acc, hi - lo);
+}
+
 struct TileArgs {
     const void *y;           // TOD in (R)
     void *z;                 // TOD out (R)
@@ -417,7 +450,12 @@ struct TileArgs {
     int L;
     const int *block_seg;    // [nb] segment of each block (-1: none), with
     const int *state;        // the PCG state per segment: stopped segments are skipped (nullptr: none)
+    MeanArgs own;            // tiles of at most 2^kFoldLog2 samples: every wave sums its block's mean
+                             // itself (see fold_means)
 };
+// Only the shorter tiles hold the code for it: in those of 32768 samples, at their
+// register limit, it cost 1.7 % even when not taken (534 -> 543 us a launch).
+constexpr int kFoldLog2 = 13;
 
 template <typename R>
 __device__ __forceinline__ void spectral_pair(R &pr, R &pi, R &qr, R &qi, Cx<R> cp, Cx<R> cq) {
@@ -464,7 +502,12 @@ __global__ __launch_bounds__((1 << LOGNC) >> LOGV, MINW) void k_tiles(TileArgs a
     R *__restrict__ z = reinterpret_cast<R *>(a.z);
     const Cx<R> *__restrict__ tw = reinterpret_cast<const Cx<R> *>(a.tw);
     const Cx<R> *__restrict__ cf = reinterpret_cast<const Cx<R> *>(a.coef) + (int64_t) d.filter * NC;
-    const R mean = (R) a.mean[d.block];
+    double mu;
+    if constexpr (LOGNC < kFoldLog2)
+        mu = a.own.partials ? wave_block_mean(a.own, d.block) : a.mean[d.block];
+    else
+        mu = a.mean[d.block];
+    const R mean = (R) mu;
     const R mean_out = (R) mean_out_of(a.edge_part, d.block, d.blk_hi - d.blk_lo);
     const int64_t in0 = d.out_lo - (a.lambda - 1);
 
@@ -1020,13 +1063,36 @@ __global__ __launch_bounds__(256) void k_block_mean(const double *__restrict__ p
     if (threadIdx.x == 0) edge_part[(int64_t) b * kEdgeSlices + sl] = part;
 }
 
-// z = y - mean over the listed (short) blocks
+// means of every block, one workgroup a block (the modes without an output mean):
+// wave k makes the lanes' sums of index k
+__global__ __launch_bounds__(64 * kMeanSums) void k_wave_mean(MeanArgs a, double *__restrict__ mean,
+                                                              const int *__restrict__ block_seg,
+                                                              const int *__restrict__ state) {
+    __shared__ double sums[kMeanSums][64];
+    const int b = (int) blockIdx.x, k = (int) (threadIdx.x >> 6), lane = (int) (threadIdx.x & 63);
+    if (state && block_seg[b] >= 0 && state[block_seg[b]]) return;  // stopped segment
+    const int64_t lo = a.start[b], hi = a.start[b + 1];
+    const int64_t last = (hi - 1) / kChunk;
+    double s = 0.0;
+#pragma unroll 4
+    for (int64_t c = lo / kChunk + (int64_t) threadIdx.x; c <= last; c += 64 * kMeanSums) s += a.partials[c + b];
+    sums[k][lane] = s;
+    __syncthreads();
+    if (k > 0) return;
+    double acc[kMeanSums];
+#pragma unroll
+    for (int j = 0; j < kMeanSums; j++) acc[j] = sums[j][lane];
+    const double mu = mean_of_sums(acc, hi - lo);
+    if (lane == 0) mean[b] = mu;
+}
+
+// z = y - mean over the listed (short) blocks; each wave sums the block's few partials itself
 template <typename R>
 __global__ void k_mean_only(const R *__restrict__ y, R *__restrict__ z, const int64_t *__restrict__ start,
-                            const int *__restrict__ blocks, const double *__restrict__ mean) {
+                            const int *__restrict__ blocks, MeanArgs a) {
     const int b = blocks[blockIdx.y];
     const int64_t lo = start[b], hi = start[b + 1];
-    const R mu = (R) mean[b];
+    const R mu = a.partials ? (R) wave_block_mean(a, b) : (R) 0;
     for (int64_t t = lo + (int64_t) blockIdx.x * blockDim.x + threadIdx.x; t < hi;
          t += (int64_t) gridDim.x * blockDim.x)
         z[t] = y[t] - mu;
@@ -1293,6 +1359,7 @@ int toeplitz_plan(Problem &pb, const int *block_sizes, int nb, int lambda, const
     for (int b = 0; b < nb; b++) {
         MGPU_ARG(block_sizes[b] > 0, "local_blocks_sizes[%d]=%d must be positive", b, block_sizes[b]);
         T.h_start[b + 1] = T.h_start[b] + block_sizes[b];
+        T.max_block = std::max(T.max_block, (int64_t) block_sizes[b]);
     }
     T.covered = T.h_start[nb];
     MGPU_ARG(T.covered <= T.m, "sum of local_blocks_sizes (%lld) exceeds m (%lld)", (long long) T.covered,
@@ -1625,7 +1692,7 @@ static TileUse tile_use(const TileClass &C, bool live) {
 
 template <typename R, int LOGNC, int LOGV, int LOGR, bool TWO, int MINW>
 static int launch_tiles_cfg(Problem &pb, const TileClass &C, const R *d_in, R *d_out, const void *coef,
-                            const void *tw, const ToeplitzScratch &sc) {
+                            const void *tw, const ToeplitzScratch &sc, const MeanArgs &own) {
     const TileUse u = tile_use<R>(C, pb.live_state != nullptr);
     if (u.ntiles == 0) return MGPU_OK;
     constexpr int NC = 1 << LOGNC, NT = NC / (1 << LOGV);
@@ -1638,7 +1705,7 @@ static int launch_tiles_cfg(Problem &pb, const TileClass &C, const R *d_in, R *d
         attr_devices.fetch_or(1u << pb.device, std::memory_order_release);
     }
     TileArgs a{d_in, d_out, u.tiles, coef, tw, sc.mean, sc.edge_part, C.lambda, u.L, pb.sg.d_block_seg,
-               pb.sg.d_block_seg ? pb.live_state : nullptr};
+               pb.sg.d_block_seg ? pb.live_state : nullptr, own};
     hipLaunchKernelGGL(kern, dim3(u.ntiles), dim3(NT), lds, pb.stream, a);
     MGPU_LAUNCHED();
     return MGPU_OK;
@@ -1660,7 +1727,7 @@ static int launch_tiles_wl(Problem &pb, const TileClass &C, const R *d_in, R *d_
         attr_devices.fetch_or(1u << pb.device, std::memory_order_release);
     }
     TileArgs a{d_in, d_out, u.tiles, coef, tw, sc.mean, sc.edge_part, C.lambda, C.L, pb.sg.d_block_seg,
-               pb.sg.d_block_seg ? pb.live_state : nullptr};
+               pb.sg.d_block_seg ? pb.live_state : nullptr, MeanArgs{}};
     hipLaunchKernelGGL(kern, dim3(u.ntiles), dim3(kWlNT), lds, pb.stream, a);
     MGPU_LAUNCHED();
     return MGPU_OK;
@@ -1668,12 +1735,12 @@ static int launch_tiles_wl(Problem &pb, const TileClass &C, const R *d_in, R *d_
 
 template <typename R>
 static int launch_tiles(Problem &pb, const TileClass &C, const R *d_in, R *d_out, int variant,
-                        const ToeplitzScratch &sc) {
+                        const ToeplitzScratch &sc, const MeanArgs &own) {
     constexpr bool F32 = sizeof(R) == 4;
     const TileUse u = tile_use<R>(C, pb.live_state != nullptr);
     const void *coef = u.coef, *tw = u.tw;
 #define MGPU_TL(LOGNC, LOGV, LOGR, TWO, MINW) \
-    return launch_tiles_cfg<R, LOGNC, LOGV, LOGR, TWO, MINW>(pb, C, d_in, d_out, coef, tw, sc)
+    return launch_tiles_cfg<R, LOGNC, LOGV, LOGR, TWO, MINW>(pb, C, d_in, d_out, coef, tw, sc, own)
     switch (u.log2n - 1) {  // LOGNC
         case 9: MGPU_TL(9, 3, 3, true, 1);
         case 10:
@@ -1796,14 +1863,14 @@ static int pick_variant(Problem &pb, TileClass &T, const R *d_in, R *d_out, cons
         const bool lng = c > nv;
         const int v = lng ? c - nv : c;
         if (two_len) T.fp32_long = lng;
-        rc = launch_tiles<R>(pb, T, d_in, d_out, v, sc);
+        rc = launch_tiles<R>(pb, T, d_in, d_out, v, sc, MeanArgs{});
         if (rc != MGPU_OK) break;
         if (hipEventRecord(e0, pb.stream) != hipSuccess) {
             set_error("tile autotuning: hipEventRecord failed");
             rc = MGPU_EHIP;
             break;
         }
-        for (int k = 0; k < 3 && rc == MGPU_OK; k++) rc = launch_tiles<R>(pb, T, d_in, d_out, v, sc);
+        for (int k = 0; k < 3 && rc == MGPU_OK; k++) rc = launch_tiles<R>(pb, T, d_in, d_out, v, sc, MeanArgs{});
         // per useful output: the two lengths have different tile counts but the same outputs
         if (rc != MGPU_OK) break;
         float ms = 0.f;
@@ -1828,6 +1895,27 @@ static int pick_variant(Problem &pb, TileClass &T, const R *d_in, R *d_out, cons
     return MGPU_OK;
 }
 
+// Whether the tiles sum their blocks' means themselves instead of a launch of
+// k_wave_mean before them (the same sums in the same order, so the same bits;
+// the symmetric mode has its edge sums to make and keeps k_block_mean).  Every
+// wave of a tile then reads its block's partials, about 1 us: less than the
+// launch (3 us and a gap) while the tiles are about one round of the chip and a
+// wave has all its loads in flight at once; with more, every round would pay.  Not where other kernels read the means, nor for
+// tiles longer than 2^kFoldLog2 samples.  (2 blocks of 4096 samples, band 64: 12.4 ->
+// 6.6 to 7.2 us a product, with the zero fill of its scratch gone too.)
+constexpr int64_t kFoldTiles = 512;
+constexpr int64_t kFoldBlock = (int64_t) 64 * kMeanSums * kChunk;  // samples of the longest block
+static bool fold_means(const ToeplitzPlan &T, bool fp32) {
+    if (!T.h_direct_blocks.empty() || T.max_block > kFoldBlock) return false;
+    int64_t tiles = 0;
+    for (const TileClass &C : T.cls) {
+        if (C.variant[fp32 ? 1 : 0] == 0) return false;  // not chosen yet: timing the variants reads the means
+        if (C.log2n > kFoldLog2 || (fp32 && C.fp32_long)) return false;
+        tiles += C.ntiles;
+    }
+    return tiles <= kFoldTiles;
+}
+
 // scratch of one product: per-chunk partial sums, block means, slice sums of
 // the symmetric mode's output mean (the plan's own buffers, or a caller's)
 template <typename R>
@@ -1842,8 +1930,8 @@ static int toeplitz_apply_t(Problem &pb, const R *d_in, R *d_out, bool compute_p
             k_partials<R><<<(unsigned) T.nchunks, 256, 0, s>>>(d_in, T.m, T.d_start, T.d_chunk_block, T.nb,
                                                                sc.partials);
             MGPU_LAUNCHED();
-            k_block_mean<R><<<dim3(T.nb, 1), 256, 0, s>>>(sc.partials, T.d_start, T.nb, sc.mean, d_in, nullptr,
-                                                          nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+            k_wave_mean<<<(unsigned) T.nb, 64 * kMeanSums, 0, s>>>(MeanArgs{sc.partials, T.d_start}, sc.mean,
+                                                                    nullptr, nullptr);
             MGPU_LAUNCHED();
             k_diag_mean<R><<<grid_for(T.m, 256), 256, 0, s>>>(d_in, d_out, T.m, T.d_start, T.nb, T.d_T0, sc.mean);
         } else {
@@ -1852,37 +1940,51 @@ static int toeplitz_apply_t(Problem &pb, const R *d_in, R *d_out, bool compute_p
         MGPU_LAUNCHED();
         return MGPU_OK;
     }
-    if (T.offset_mode != MGPU_OFFSET_NONE) {  // MGPU_OFFSET_NONE: means stay 0
+    MeanArgs own{}, shrt{};  // for the tiles (fold_means) and the short blocks
+    ToeplitzScratch use = sc;
+    const bool sym = T.offset_mode == MGPU_OFFSET_SYMMETRIC;
+    if (!sym) use.edge_part = T.d_edge_part;  // the plan's, zero in the other modes
+    if (T.offset_mode == MGPU_OFFSET_NONE) {
+        use.mean = T.d_mean;  // the plan's, zero in this mode
+    } else {
         pb.prof.begin(MGPU_KT_MEAN, s);
         if (compute_partials) {
             k_partials<R><<<(unsigned) T.nchunks, 256, 0, s>>>(d_in, T.m, T.d_start, T.d_chunk_block, T.nb,
                                                                sc.partials);
             MGPU_LAUNCHED();
         }
-        const bool sym = T.offset_mode == MGPU_OFFSET_SYMMETRIC;
-        k_block_mean<R><<<dim3(T.nb, sym ? kEdgeSlices : 1), 256, 0, s>>>(
-                sc.partials, T.d_start, T.nb, sc.mean, d_in, T.d_tail, T.d_tail_off, T.d_block_filter, T.d_block_kind,
-                T.d_block_lambda,
-                sym ? sc.edge_part : nullptr, pb.sg.d_block_seg, pb.sg.d_block_seg ? pb.live_state : nullptr);
-        MGPU_LAUNCHED();
+        const int *seg = pb.sg.d_block_seg, *live = seg ? pb.live_state : nullptr;
+        shrt = MeanArgs{sc.partials, T.d_start};
+        if (sym) {
+            k_block_mean<R><<<dim3(T.nb, kEdgeSlices), 256, 0, s>>>(
+                    sc.partials, T.d_start, T.nb, sc.mean, d_in, T.d_tail, T.d_tail_off, T.d_block_filter,
+                    T.d_block_kind, T.d_block_lambda, sc.edge_part, seg, live);
+            MGPU_LAUNCHED();
+        } else if (fold_means(T, sizeof(R) == 4)) {
+            own = shrt;
+        } else {
+            k_wave_mean<<<(unsigned) T.nb, 64 * kMeanSums, 0, s>>>(shrt, sc.mean, seg, live);
+            MGPU_LAUNCHED();
+        }
         pb.prof.end(s);
     }
     // one launch per tile class (band and tile length), in one profiled span
-    for (TileClass &C : T.cls) MGPU_RET(pick_variant<R>(pb, C, d_in, d_out, sc));
+    for (TileClass &C : T.cls) MGPU_RET(pick_variant<R>(pb, C, d_in, d_out, use));
     if (!T.cls.empty()) {
         pb.prof.begin(MGPU_KT_TILES, s);
-        for (TileClass &C : T.cls) MGPU_RET(launch_tiles<R>(pb, C, d_in, d_out, C.variant[sizeof(R) == 4 ? 1 : 0], sc));
+        for (TileClass &C : T.cls)
+            MGPU_RET(launch_tiles<R>(pb, C, d_in, d_out, C.variant[sizeof(R) == 4 ? 1 : 0], use, own));
         pb.prof.end(s);
     }
     if (!T.h_direct_blocks.empty()) {
         k_direct<R><<<dim3(64, (unsigned) T.h_direct_blocks.size()), 256, 0, s>>>(
-                d_in, d_out, T.d_start, T.d_direct_blocks, sc.mean, sc.edge_part, T.d_direct_invtt, T.d_inv_off,
+                d_in, d_out, T.d_start, T.d_direct_blocks, use.mean, use.edge_part, T.d_direct_invtt, T.d_inv_off,
                 T.d_block_lambda);
         MGPU_LAUNCHED();
     }
     if (!T.h_short_blocks.empty()) {
         k_mean_only<R><<<dim3(16, (unsigned) T.h_short_blocks.size()), 256, 0, s>>>(d_in, d_out, T.d_start,
-                                                                                  T.d_short_blocks, sc.mean);
+                                                                                  T.d_short_blocks, shrt);
         MGPU_LAUNCHED();
     }
     if (T.covered < T.m) {
@@ -1911,11 +2013,6 @@ int toeplitz_apply_f32(Problem &pb, const float *d_in, float *d_out, bool comput
 
 size_t toeplitz_scratch_doubles(const ToeplitzPlan &T) {
     return (size_t) (T.nchunks + T.nb) + (size_t) T.nb + (size_t) T.nb * kEdgeSlices;
-}
-
-__global__ void k_fill_zero(double *__restrict__ p, int64_t n) {
-    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1979,14 +2076,6 @@ int toeplitz_apply_scratch(Problem &pb, const double *d_in, double *d_out, doubl
     sc.partials = d_scratch;
     sc.mean = sc.partials + (T.nchunks + T.nb);
     sc.edge_part = sc.mean + T.nb;
-    // means and output-mean slices that the product reads but no kernel of this
-    // mode writes must be zero (the array keeps the previous call's values):
-    // cleared with a kernel so that a captured graph holds no memset node
-    const int64_t nz = (int64_t) T.nb * (1 + kEdgeSlices);
-    if (T.lambda > 1 && T.offset_mode != MGPU_OFFSET_SYMMETRIC) {
-        k_fill_zero<<<grid_for(nz, 256), 256, 0, pb.stream>>>(sc.mean, nz);
-        MGPU_LAUNCHED();
-    }
     return toeplitz_apply_t<double>(pb, d_in, d_out, true, sc);
 }
 
