@@ -460,8 +460,9 @@ struct TwoLevel {
     double *d_AZ = nullptr;     // [zn * ld]
     double *d_Em1 = nullptr;    // [zn * zn] row-major
     double *d_qtx = nullptr;    // [zn] Em1 Z^T g of the last apply
-    double *d_part = nullptr;   // [zn * nchunk] partials of Z^T g
-    int nchunk = 0;
+    double *d_part = nullptr;   // [zn * nzt] partials of Z^T g
+    int nzt = 0, zt_len = 0;    // chunks of Z^T g and their length
+    int nchunk = 0;             // chunks of the dots of the build
     double build_ms = 0.0;      // device time of the last build
 };
 

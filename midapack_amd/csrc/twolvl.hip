@@ -16,10 +16,11 @@
 // Device layout: Z and A Z are column-major (column j contiguous, stride
 // 3 npix), so Z^T g is Zn coalesced dot products and Z Qtx / AZ Qtx are
 // per-pixel combinations fused with the 3x3 block-Jacobi product and the PCG
-// dots.  Per PCG iteration the preconditioner costs three launches: partial
-// dots of Z^T g (chunks x Zn workgroups), one workgroup that sums them in a
-// fixed order and multiplies by Em1, and the fused apply, which reads Z and
-// A Z once.  All sums run in a fixed order, so results are deterministic.
+// dots.  Per PCG iteration the preconditioner costs two launches: partial dots
+// of Z^T g (chunks x Zn workgroups) and the fused apply, which reads Z and A Z
+// once and whose workgroups sum the partials and multiply by Em1 themselves;
+// with many columns or a large map one workgroup does that in a launch between
+// them (see twolvl_apply).  All sums run in a fixed order, so results are deterministic.
 // The Zn x Zn work (pinv of E, eigenvectors of the Lanczos tridiagonal) runs
 // on the host: Zn is at most kMaxZn.
 #include "pcg_device.h"
@@ -147,51 +148,81 @@ __global__ __launch_bounds__(256) void k_combine(const double *__restrict__ in, 
     out[(int64_t) j * ld + i] = s;
 }
 
-// Z^T g partials: block (c, j) sums Z_j[k] g[k] over chunk c (build_Qtx,
-// precond.c:1043-1046, pixpond = 1 on one rank)
+// Z^T g partials: block (c, j) sums Z_j[k] g[k] over chunk c of len entries
+// (build_Qtx, precond.c:1043-1046, pixpond = 1 on one rank).  Bound by the
+// latency of its loads while Z comes from the last-level cache: kZtPer products
+// a thread are loaded at once, and a chunk is one round of them until the map
+// has kZtParts chunks (65536 pixels, 8 columns: 24 us with one load in flight and
+// chunks of 16384, 5.0 now).
+constexpr int kZtPer = 8, kZtParts = 256;
 __global__ __launch_bounds__(kZB) void k_zt_part(const double *__restrict__ Z, int64_t ld, int n,
                                                  const double *__restrict__ g, double *__restrict__ part, int nchunk,
-                                                 const int *__restrict__ state, const int *__restrict__ flag) {
+                                                 int len, const int *__restrict__ state,
+                                                 const int *__restrict__ flag) {
     if (flag && stopped(flag)) return;
     if (state && state[0]) return;
     __shared__ double red[kZB / 64];
     const int j = blockIdx.y;
     const double *z = Z + (int64_t) j * ld;
-    const int k0 = blockIdx.x * kZChunk, k1 = min(n, k0 + kZChunk);
+    const int64_t k0 = (int64_t) blockIdx.x * len, k1 = min((int64_t) n, k0 + len);
     double s = 0.0;
-    for (int k = k0 + (int) threadIdx.x; k < k1; k += kZB) s += z[k] * g[k] * 1.0;
+    for (int64_t k = k0 + (int) threadIdx.x; k < k1; k += kZB * kZtPer) {
+        double a[kZtPer], b[kZtPer];
+#pragma unroll
+        for (int u = 0; u < kZtPer; u++) {
+            const bool in = k + u * kZB < k1;
+            a[u] = in ? z[k + u * kZB] : 0.0;
+            b[u] = in ? g[k + u * kZB] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kZtPer; u++)
+            if (k + u * kZB < k1) s += a[u] * b[u] * 1.0;
+    }
     s = block_sum(s, red);
     if (threadIdx.x == 0) part[(int64_t) j * nchunk + blockIdx.x] = s;
 }
 
-// w = Z^T g summed over chunks in order, Qtx = Em1 w (precond.c:1050-1054)
+// w = Z^T g summed over chunks in a fixed order by one wave a column,
+// qs = Em1 w (precond.c:1050-1054); kZB threads, w and qs in LDS
+__device__ __forceinline__ void zt_sum(const double *__restrict__ part, int nchunk, int zn,
+                                       const double *__restrict__ Em1, double *w, double *qs) {
+    for (int j = (int) (threadIdx.x >> 6); j < zn; j += kZB / 64) {
+        double s = 0.0;
+#pragma unroll 4
+        for (int c = (int) (threadIdx.x & 63); c < nchunk; c += 64) s += part[(int64_t) j * nchunk + c];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if ((threadIdx.x & 63) == 0) w[j] = s;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < zn) {
+        double qv = 0.0;
+#pragma unroll 4
+        for (int j = 0; j < zn; j++) qv += Em1[t * zn + j] * w[j];
+        qs[t] = qv;
+    }
+}
+
 __global__ __launch_bounds__(kZB) void k_zt_fin(const double *__restrict__ part, int nchunk, int zn,
                                                 const double *__restrict__ Em1, double *__restrict__ qtx,
                                                 const int *__restrict__ state, const int *__restrict__ flag) {
     if (flag && stopped(flag)) return;
     if (state && state[0]) return;
     __shared__ double w[kMaxZn];
-    const int t = threadIdx.x;
-    if (t < zn) {
-        double s = 0.0;
-        for (int c = 0; c < nchunk; c++) s += part[(int64_t) t * nchunk + c];
-        w[t] = s;
-    }
-    __syncthreads();
-    if (t < zn) {
-        double qv = 0.0;
-        for (int j = 0; j < zn; j++) qv += Em1[t * zn + j] * w[j];
-        qtx[t] = qv;
-    }
+    zt_sum(part, nchunk, zn, Em1, w, qtx);
 }
+static_assert(kMaxZn <= kZB && kZB == kMB, "zt_sum: a thread per column, in both kernels");
 
 // Cg = BJ (g - AZ Qtx) + Z Qtx for the pixels of the workgroup, then the PCG
-// dot partials: INIT: h = Cg, [<Cg,g> | <g,g>]; else [<Cg,g> | <Cg,g-gp> | <g,g>]
-template <bool INIT>
+// dot partials: INIT: h = Cg, [<Cg,g> | <g,g>]; else [<Cg,g> | <Cg,g-gp> | <g,g>].
+// SUM: Qtx summed here from the partials of Z^T g (zt_sum), else read.  Four
+// columns' 24 loads are in flight at once (65536 pixels, 8 columns: 10.3 us with
+// one column's and Qtx from k_zt_fin, 4.7 us more; 10.9 now with SUM).
+template <bool INIT, bool SUM>
 __global__ __launch_bounds__(kMB) void k_twolvl_apply(
         const double *__restrict__ Z, const double *__restrict__ AZ, int64_t ld, int zn,
-        const double *__restrict__ qtx, const double *__restrict__ inv, const double *__restrict__ g,
-        const double *__restrict__ gp, double *__restrict__ Cg, double *__restrict__ h,
+        const double *__restrict__ qtx, const double *__restrict__ zpart, int nzt, const double *__restrict__ Em1,
+        const double *__restrict__ inv, const double *__restrict__ g, const double *__restrict__ gp, double *__restrict__ Cg, double *__restrict__ h,
         const int *__restrict__ wg_seg, const int *__restrict__ wg_q0, const int *__restrict__ seg_q,
         const int *__restrict__ state, double *__restrict__ part, const int *__restrict__ flag) {
     if (flag && stopped(flag)) return;
@@ -199,22 +230,28 @@ __global__ __launch_bounds__(kMB) void k_twolvl_apply(
     if (state && state[sp.r]) return;  // uniform over the workgroup
     __shared__ double red[kMB / 64];
     __shared__ double qs[kMaxZn];
-    for (int j = threadIdx.x; j < zn; j += kMB) qs[j] = qtx[j];
+    if constexpr (SUM) {
+        __shared__ double w[kMaxZn];
+        zt_sum(zpart, nzt, zn, Em1, w, qs);
+    } else {
+        for (int j = threadIdx.x; j < zn; j += kMB) qs[j] = qtx[j];
+    }
     __syncthreads();
     const int q = sp.q;
     double a = 0.0, b = 0.0, c = 0.0;
     if (q < sp.qend) {
-        double qg[3], r[3], gv[3];
-        for (int e = 0; e < 3; e++) {
-            const int64_t i = 3 * (int64_t) q + e;
-            double zq = 0.0, azq = 0.0;  // mul_ZQtx: vec[k] += Z[j][k] Qtx[j], j ascending
-            for (int j = 0; j < zn; j++) {
-                zq += Z[(int64_t) j * ld + i] * qs[j];
-                azq += AZ[(int64_t) j * ld + i] * qs[j];
+        double qg[3] = {}, azq[3] = {}, r[3], gv[3];
+        const int64_t i = 3 * (int64_t) q;
+        // mul_ZQtx: vec[k] += Z[j][k] Qtx[j], j ascending
+#pragma unroll 4
+        for (int j = 0; j < zn; j++)
+            for (int e = 0; e < 3; e++) {
+                qg[e] += Z[(int64_t) j * ld + i + e] * qs[j];
+                azq[e] += AZ[(int64_t) j * ld + i + e] * qs[j];
             }
-            gv[e] = g[i];
-            qg[e] = zq;
-            r[e] = gv[e] - azq;
+        for (int e = 0; e < 3; e++) {
+            gv[e] = g[i + e];
+            r[e] = gv[e] - azq[e];
         }
         const double *M = inv + 9 * (int64_t) q;
         for (int e = 0; e < 3; e++) {
@@ -475,10 +512,12 @@ int twolvl_build(Problem &pb, const double *d_signal, const double *d_noise) {
     T.zn = zn;
     T.ld = n;
     T.nchunk = (int) ((n + kZChunk - 1) / kZChunk);
+    T.zt_len = kZB * kZtPer * (int) grid_for(n, (int64_t) kZB * kZtPer * kZtParts);
+    T.nzt = (int) grid_for(n, T.zt_len);
     const int64_t ld = T.ld;
     MGPU_RET(pb.arena.alloc(&T.d_Em1, (size_t) zn * zn));
     MGPU_RET(pb.arena.alloc(&T.d_qtx, (size_t) zn));
-    MGPU_RET(pb.arena.alloc(&T.d_part, (size_t) zn * T.nchunk));
+    MGPU_RET(pb.arena.alloc(&T.d_part, (size_t) zn * T.nzt));
     MGPU_RET(pb.arena.alloc(&T.d_Z, (size_t) zn * ld));
     MGPU_RET(pb.arena.alloc(&T.d_AZ, (size_t) zn * ld));
     if (precond == 1) {
@@ -533,6 +572,8 @@ int twolvl_build(Problem &pb, const double *d_signal, const double *d_noise) {
     return MGPU_OK;
 }
 
+constexpr int kSumZn = 16, kSumWgs = 512;
+
 int twolvl_apply(Problem &pb, const double *d_g, const double *d_gp, double *d_Cg, double *d_h, double *d_part,
                  bool init, const int *d_state, const int *d_flag) {
     const TwoLevel &T = pb.tl;
@@ -540,17 +581,20 @@ int twolvl_apply(Problem &pb, const double *d_g, const double *d_gp, double *d_C
     hipStream_t s = pb.stream;
     const int n = 3 * pb.pt.npix;
     MGPU_ARG(T.zn > 0 && T.ld == n, "two-level preconditioner not built for this map");
-    k_zt_part<<<dim3(T.nchunk, T.zn), kZB, 0, s>>>(T.d_Z, T.ld, n, d_g, T.d_part, T.nchunk, d_state, d_flag);
+    k_zt_part<<<dim3(T.nzt, T.zn), kZB, 0, s>>>(T.d_Z, T.ld, n, d_g, T.d_part, T.nzt, T.zt_len, d_state, d_flag);
     MGPU_LAUNCHED();
-    k_zt_fin<<<1, kZB, 0, s>>>(T.d_part, T.nchunk, T.zn, T.d_Em1, T.d_qtx, d_state, d_flag);
-    MGPU_LAUNCHED();
-    if (init)
-        k_twolvl_apply<true><<<G.nwg, kMB, 0, s>>>(T.d_Z, T.d_AZ, T.ld, T.zn, T.d_qtx, pb.pc.d_inv, d_g, d_gp, d_Cg,
-                                                   d_h, G.d_wg_seg, G.d_wg_q0, G.d_q, d_state, d_part, d_flag);
-    else
-        k_twolvl_apply<false><<<G.nwg, kMB, 0, s>>>(T.d_Z, T.d_AZ, T.ld, T.zn, T.d_qtx, pb.pc.d_inv, d_g, d_gp,
-                                                    d_Cg, d_h, G.d_wg_seg, G.d_wg_q0, G.d_q, d_state, d_part,
-                                                    d_flag);
+    // Every workgroup of the apply reads the zn * nzt partials and Em1 again: less
+    // than a launch while the columns are few and the workgroups about one round of
+    // the chip (8 columns, 256 workgroups: 1 us against 4.7); past that k_zt_fin reads them once.
+    const bool sum = T.zn <= kSumZn && G.nwg <= kSumWgs;
+    if (!sum) {
+        k_zt_fin<<<1, kZB, 0, s>>>(T.d_part, T.nzt, T.zn, T.d_Em1, T.d_qtx, d_state, d_flag);
+        MGPU_LAUNCHED();
+    }
+    auto k = init ? sum ? k_twolvl_apply<true, true> : k_twolvl_apply<true, false>
+                  : sum ? k_twolvl_apply<false, true> : k_twolvl_apply<false, false>;
+    k<<<G.nwg, kMB, 0, s>>>(T.d_Z, T.d_AZ, T.ld, T.zn, T.d_qtx, T.d_part, T.nzt, T.d_Em1, pb.pc.d_inv, d_g, d_gp,
+                            d_Cg, d_h, G.d_wg_seg, G.d_wg_q0, G.d_q, d_state, d_part, d_flag);
     MGPU_LAUNCHED();
     return MGPU_OK;
 }
