@@ -13,8 +13,8 @@
 //     the local pixels of item r are one contiguous range, a map segment of the
 //     PCG (pcg.hip) with its own tolerance and iteration cap.
 //   * Toeplitz blocks keep their item's band and the tile length the item would
-//     use alone: the plan holds one tile class per (band, tile length), and an
-//     N^-1 product launches one tile kernel per class, all in the same launch
+//     use alone: the plan holds one tile class per (band, tile length); an
+//     N^-1 product launches the short-tile classes together, all in the same launch
 //     sequence of each PCG iteration.
 // P, N^-1 and P^T are block diagonal over the items, the preconditioner and
 // the cut are per pixel and the PCG scalars are per segment, so each item

@@ -478,8 +478,8 @@ __device__ __forceinline__ void spectral_self(R &pr, R &pi, Cx<R> c) {
     pi = npi;
 }
 
-template <typename R, int LOGNC, int LOGV, int LOGR, bool TWO, int MINW>
-__global__ __launch_bounds__((1 << LOGNC) >> LOGV, MINW) void k_tiles(TileArgs a) {
+template <typename R, int LOGNC, int LOGV, int LOGR, bool TWO>
+__device__ __forceinline__ void tile_product(const TileArgs &a, int tile) {
     constexpr int NC = 1 << LOGNC, V = 1 << LOGV, NT = NC / V;
     constexpr int NP = n_passes(LOGNC, LOGV, LOGR);
     constexpr int LR0 = fwd_bits(LOGNC, LOGV, LOGR, 0);
@@ -493,7 +493,7 @@ __global__ __launch_bounds__((1 << LOGNC) >> LOGV, MINW) void k_tiles(TileArgs a
     R *lds = reinterpret_cast<R *>(smem_raw);
 
     const int t = threadIdx.x;
-    const TileDesc d = a.tiles[blockIdx.x];
+    const TileDesc d = a.tiles[tile];
     if (a.state) {  // the tile's segment has stopped (uniform over the workgroup)
         const int sg = a.block_seg[d.block];
         if (sg >= 0 && a.state[sg]) return;
@@ -657,6 +657,41 @@ __global__ __launch_bounds__((1 << LOGNC) >> LOGV, MINW) void k_tiles(TileArgs a
         }
     }
     (void) NP;
+}
+
+template <typename R, int LOGNC, int LOGV, int LOGR, bool TWO, int MINW>
+__global__ __launch_bounds__((1 << LOGNC) >> LOGV, MINW) void k_tiles(TileArgs a) {
+    tile_product<R, LOGNC, LOGV, LOGR, TWO>(a, (int) blockIdx.x);
+}
+
+// The tiles of several classes (bands, tile lengths) in one launch, each computed
+// as k_tiles' default variant of its length does: the same bits.  The classes of a
+// batch of small maps have a few hundred tiles each, less than a round of the
+// chip, and their launches would run one after the other (see launch_multi).
+// A workgroup has the threads of the longest tile; waves beyond its own tile's end
+// at once, which a barrier does not wait for.  Three waves a SIMD as k_tiles has
+// (27 registers spilled; two waves and none: the same times).
+constexpr int kMultiMax = 16, kMultiLog2Min = 10, kMultiLog2Max = 13;
+struct MultiArgs {
+    int n;
+    int first[kMultiMax];   // class k's workgroups start at first[k]
+    int lognc[kMultiMax];
+    TileArgs cls[kMultiMax];
+};
+template <typename R>
+__global__ __launch_bounds__(256, 3) void k_tiles_multi(MultiArgs m) {
+    int k = 0;
+    while (k + 1 < m.n && (int) blockIdx.x >= m.first[k + 1]) k++;
+    const int tile = (int) blockIdx.x - m.first[k], lognc = m.lognc[k];
+    const int wave = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
+    if (wave >= ((1 << lognc) >> (lognc == 9 ? 3 : 4)) / 64) return;
+    switch (lognc) {
+        case 9: tile_product<R, 9, 3, 3, true>(m.cls[k], tile); break;
+        case 10: tile_product<R, 10, 4, 4, false>(m.cls[k], tile); break;
+        case 11: tile_product<R, 11, 4, 4, false>(m.cls[k], tile); break;
+        case 12: tile_product<R, 12, 4, 4, false>(m.cls[k], tile); break;
+        default: break;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1916,6 +1951,54 @@ static bool fold_means(const ToeplitzPlan &T, bool fp32) {
     return tiles <= kFoldTiles;
 }
 
+// Launches the classes' tiles together (k_tiles_multi) where that pays: at least
+// two classes of the default variant with tiles of 1024 to 8192 samples; done[c] is
+// set for those.  12 maps of 3 tile lengths: 11.5 + 10.8 + 7.8 us as three launches,
+// 16.6 us as one; the batch 4.43 -> 4.07 ms.  The gain fades as the classes fill the
+// chip by themselves (100 iterations of 24 maps 11.3 -> 10.8 ms, of 96 maps 34.9 ->
+// 34 ms, of 24 larger maps with about 7000 tiles 28.6 -> 27.3 ms): beyond the sizes
+// measured a class keeps its own kernel, which needs no registers for the others.
+constexpr int64_t kMultiTiles = 8192;
+template <typename R>
+static int launch_multi(Problem &pb, const R *d_in, R *d_out, const ToeplitzScratch &sc, const MeanArgs &own,
+                        std::vector<char> &done) {
+    constexpr bool F32 = sizeof(R) == 4;
+    const ToeplitzPlan &T = pb.tp;
+    std::vector<int> pick;
+    int64_t tiles = 0;
+    for (size_t c = 0; c < T.cls.size(); c++) {
+        const TileUse u = tile_use<R>(T.cls[c], pb.live_state != nullptr);
+        if (u.log2n < kMultiLog2Min || u.log2n > kMultiLog2Max || u.ntiles == 0 ||
+            T.cls[c].variant[F32 ? 1 : 0] != default_variant(F32, u.log2n))
+            continue;
+        pick.push_back((int) c);
+        tiles += u.ntiles;
+    }
+    if (pick.size() < 2 || tiles > kMultiTiles) return MGPU_OK;
+    const int *seg = pb.sg.d_block_seg;
+    for (size_t p0 = 0; p0 < pick.size(); p0 += kMultiMax) {
+        MultiArgs m{};
+        int grid = 0, threads = 0;
+        size_t lds = 0;
+        for (size_t p = p0; p < std::min(pick.size(), p0 + kMultiMax); p++) {
+            const TileClass &C = T.cls[pick[p]];
+            const TileUse u = tile_use<R>(C, pb.live_state != nullptr);
+            const int lognc = u.log2n - 1;
+            m.first[m.n] = grid;
+            m.lognc[m.n] = lognc;
+            m.cls[m.n++] = TileArgs{d_in, d_out, u.tiles, u.coef, u.tw, sc.mean, sc.edge_part, C.lambda, u.L, seg,
+                                    seg ? pb.live_state : nullptr, own};
+            grid += u.ntiles;
+            threads = std::max(threads, (1 << lognc) >> (lognc == 9 ? 3 : 4));
+            lds = std::max(lds, sizeof(R) * (size_t) lds_elems(1 << lognc) * (lognc == 9 ? 2 : 1));
+            done[pick[p]] = 1;
+        }
+        k_tiles_multi<R><<<(unsigned) grid, threads, lds, pb.stream>>>(m);
+        MGPU_LAUNCHED();
+    }
+    return MGPU_OK;
+}
+
 // scratch of one product: per-chunk partial sums, block means, slice sums of
 // the symmetric mode's output mean (the plan's own buffers, or a caller's)
 template <typename R>
@@ -1968,12 +2051,16 @@ static int toeplitz_apply_t(Problem &pb, const R *d_in, R *d_out, bool compute_p
         }
         pb.prof.end(s);
     }
-    // one launch per tile class (band and tile length), in one profiled span
+    // one launch per tile class (band and tile length) or of several classes, in one
+    // profiled span
     for (TileClass &C : T.cls) MGPU_RET(pick_variant<R>(pb, C, d_in, d_out, use));
     if (!T.cls.empty()) {
         pb.prof.begin(MGPU_KT_TILES, s);
-        for (TileClass &C : T.cls)
-            MGPU_RET(launch_tiles<R>(pb, C, d_in, d_out, C.variant[sizeof(R) == 4 ? 1 : 0], use, own));
+        std::vector<char> done(T.cls.size(), 0);
+        MGPU_RET(launch_multi<R>(pb, d_in, d_out, use, own, done));
+        for (size_t c = 0; c < T.cls.size(); c++)
+            if (!done[c])
+                MGPU_RET(launch_tiles<R>(pb, T.cls[c], d_in, d_out, T.cls[c].variant[sizeof(R) == 4 ? 1 : 0], use, own));
         pb.prof.end(s);
     }
     if (!T.h_direct_blocks.empty()) {
