@@ -70,6 +70,30 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
     return s;
 }
 
+// three block_sums at once, with their bits (red: 3 * blockDim.x / 64 doubles)
+__device__ __forceinline__ void block_sum3(double &a, double &b, double &c, double *red) {
+    const int W = (int) (blockDim.x >> 6), w = (int) (threadIdx.x >> 6);
+    for (int o = 32; o > 0; o >>= 1) {
+        a += __shfl_xor(a, o);
+        b += __shfl_xor(b, o);
+        c += __shfl_xor(c, o);
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+        red[w] = a;
+        red[W + w] = b;
+        red[2 * W + w] = c;
+    }
+    __syncthreads();
+    a = b = c = 0.0;
+    if (threadIdx.x == 0)
+        for (int i = 0; i < W; i++) {
+            a += red[i];
+            b += red[W + i];
+            c += red[2 * W + i];
+        }
+}
+
 // threads of the scalar reductions (one workgroup per segment)
 constexpr int kRB = 1024;
 
@@ -103,6 +127,7 @@ template <int NS>
 __device__ __forceinline__ void reduce_parts_wg(const double *__restrict__ p, int64_t stride, int nparts, double *red,
                                                 double (&out)[NS]) {
     constexpr int J = kRB / kMB, W = kRB / 64;
+    const int w0 = __builtin_amdgcn_readfirstlane((int) threadIdx.x & ~63);  // the wave's first thread
     double v[NS][J];
 #pragma unroll
     for (int k = 0; k < NS; k++)
@@ -116,7 +141,8 @@ __device__ __forceinline__ void reduce_parts_wg(const double *__restrict__ p, in
 #pragma unroll
         for (int j = 0; j < J; j++) {
             double s = 0.0 + v[k][j];
-            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+            if (w0 + j * kMB < nparts)  // a wave without partials has the sum +0.0
+                for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
             if ((threadIdx.x & 63) == 0) red[k * W + (threadIdx.x >> 6) + j * (kMB / 64)] = s;
         }
     __syncthreads();
