@@ -109,72 +109,84 @@ struct TrArgs {
 // per class, took 101 us.  (Four detectors a workgroup, for fewer loads of the
 // weights, leave fewer waves to hide it: 61 us.)
 template <int NP, int NH>
-__global__ __launch_bounds__(256) void k_tmpl_part(TrArgs a) {
+__global__ __launch_bounds__(256, NP <= 1 && NH <= 2 ? 8 : 1) void k_tmpl_part(TrArgs a) {
     if (a.state && *a.state) return;  // the solve has stopped: queued iterations do no work
     __shared__ double sv[kTChunk];
     // workgroup b runs on XCD b % 8: each XCD gets a contiguous run of (chunk, detector)
     const int n_all = a.nchunks * a.ndet, x = (int) blockIdx.x & 7, rem = n_all & 7;
     const int idx = x * (n_all >> 3) + min(x, rem) + ((int) blockIdx.x >> 3);
     const int chunk = idx / a.ndet, c = a.chunk_ces[chunk], b = c * a.ndet + idx % a.ndet, lo = a.chunk_lo[chunk];
+    const int p0 = a.chunk_p[chunk], np = a.chunk_p[chunk + 1] - p0, h0 = a.chunk_h[chunk],
+              nh = a.chunk_h[chunk + 1] - h0, nall = np + nh + a.nsss;
+    const int lane = threadIdx.x & 15, grp = (int) threadIdx.x >> 4;
+    // start (of the CES; azimuth bins: in the chunk's order) and length of item k
+    auto item = [&](int k) {
+        if (k < np) return a.ppiece[p0 + k];
+        if (k < np + nh) return a.hpiece[h0 + k - np];
+        if (k >= nall) return make_int2(0, 0);
+        const unsigned short *__restrict__ ab = a.abin + (int64_t) chunk * (a.nsss + 1) + (k - np - nh);
+        return make_int2(ab[0], ab[1] - ab[0]);
+    };
+    int2 ahead = item(grp + 16 * lane);  // lane l of a group: its item of round l
     const int n = min(kTChunk, a.len[c] - lo);
     const int64_t cb = a.c0[c];
     const double sc = a.scale ? a.scale[b] : 1.0;
     const double *__restrict__ yb = a.y + a.start[b] + lo;
+    const TPieces P = a.pieces[c];
+    double *__restrict__ op = a.part + a.poff[b], *__restrict__ oh = op + (int64_t) a.npoly * P.np;
+    double *__restrict__ oa = oh + (int64_t) a.nh2 * P.nh + (int64_t) (chunk - P.ch0) * a.nsss;
 #pragma unroll
     for (int k = 0; k < kTChunk / 256; k++) {
         const int i = (int) threadIdx.x + k * 256;
         if (i < n) sv[i] = sc * yb[i];
     }
     __syncthreads();
-    const int lane = threadIdx.x & 15;
-    const TPieces P = a.pieces[c];
-    double *__restrict__ op = a.part + a.poff[b], *__restrict__ oh = op + (int64_t) a.npoly * P.np;
-    double *__restrict__ oa = oh + (int64_t) a.nh2 * P.nh + (int64_t) (chunk - P.ch0) * a.nsss;
-    const int p0 = a.chunk_p[chunk], np = a.chunk_p[chunk + 1] - p0, h0 = a.chunk_h[chunk],
-              nh = a.chunk_h[chunk + 1] - h0;
-    for (int k = threadIdx.x >> 4; k < np + nh + a.nsss; k += 16) {
+    // an item's sum of w[o] v over its samples, in sample order: lane l takes l, l + 16,
+    // ...; a piece is one round of loads with up to two weights a sample, two with four
+    auto sums = [&](const double *__restrict__ w, const double *v, int len, int no, auto &acc) {
+        constexpr int N = sizeof(acc) / sizeof(double), U = N <= 2 ? kTPiece / 16 : N <= 4 ? 4 : 1;
+#pragma unroll
+        for (int o = 0; o < N; o++) acc[o] = 0.0;
+        for (int i0 = lane; i0 - lane < len; i0 += 16 * U) {
+            double wv[U][N];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = min(i0 + 16 * u, len - 1);
+#pragma unroll
+                for (int o = 0; o < N; o++) wv[u][o] = o < no ? w[o * a.ncs + i] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (i0 + 16 * u < len)
+#pragma unroll
+                    for (int o = 0; o < N; o++)
+                        if (o < no) acc[o] += wv[u][o] * v[i0 + 16 * u];
+        }
+#pragma unroll
+        for (int o = 0; o < N; o++) acc[o] = sum16(acc[o]);
+    };
+    for (int k = grp, rd = 0; k < nall; k += 16, rd = (rd + 1) & 15) {
+        if (rd == 0 && k > grp) ahead = item(k + 16 * lane);
+        const int2 pc = make_int2(__shfl(ahead.x, rd, 16), __shfl(ahead.y, rd, 16));
         if (k < np) {
-            const int2 pc = a.ppiece[p0 + k];
-            const double *__restrict__ w = a.leg + cb + pc.x, *v = sv + (pc.x - lo);
             double acc[NP];
+            sums(a.leg + cb + pc.x, sv + (pc.x - lo), pc.y, a.npoly, acc);
 #pragma unroll
-            for (int o = 0; o < NP; o++) acc[o] = 0.0;
-#pragma unroll 4
-            for (int i = lane; i < pc.y; i += 16)
-#pragma unroll
-                for (int o = 0; o < NP; o++)
-                    if (o < a.npoly) acc[o] += w[o * a.ncs + i] * v[i];
-#pragma unroll
-            for (int o = 0; o < NP; o++) {
-                const double s = sum16(acc[o]);
-                if (o < a.npoly && lane == 0) op[(int64_t) (p0 - P.p0 + k) * a.npoly + o] = s;
-            }
+            for (int o = 0; o < NP; o++)
+                if (o < a.npoly && lane == 0) op[(int64_t) (p0 - P.p0 + k) * a.npoly + o] = acc[o];
         } else if (k < np + nh) {
-            const int2 pc = a.hpiece[h0 + k - np];
-            const double *__restrict__ w = a.hc + cb + pc.x, *v = sv + (pc.x - lo);
             double acc[NH];
+            sums(a.hc + cb + pc.x, sv + (pc.x - lo), pc.y, a.nh2, acc);
 #pragma unroll
-            for (int h = 0; h < NH; h++) acc[h] = 0.0;
-#pragma unroll 4
-            for (int i = lane; i < pc.y; i += 16)
-#pragma unroll
-                for (int h = 0; h < NH; h++)
-                    if (h < a.nh2) acc[h] += w[h * a.ncs + i] * v[i];
-#pragma unroll
-            for (int h = 0; h < NH; h++) {
-                const double s = sum16(acc[h]);
-                if (h < a.nh2 && lane == 0) oh[(int64_t) (h0 - P.h0 + k - np) * a.nh2 + h] = s;
-            }
+            for (int h = 0; h < NH; h++)
+                if (h < a.nh2 && lane == 0) oh[(int64_t) (h0 - P.h0 + k - np) * a.nh2 + h] = acc[h];
         } else {
-            const int q = k - np - nh;
-            const unsigned short *__restrict__ ab = a.abin + (int64_t) chunk * (a.nsss + 1) + q;
-            const unsigned short *__restrict__ ord = a.order + cb + lo;
-            const int e = ab[1];
+            const unsigned short *__restrict__ ord = a.order + cb + lo + pc.x;
             double acc = 0.0;
 #pragma unroll 4
-            for (int i = ab[0] + lane; i < e; i += 16) acc += sv[ord[i]];
+            for (int i = lane; i < pc.y; i += 16) acc += sv[ord[i]];
             acc = sum16(acc);
-            if (lane == 0) oa[q] = acc;
+            if (lane == 0) oa[k - np - nh] = acc;
         }
     }
 }
