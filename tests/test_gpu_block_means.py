@@ -58,3 +58,21 @@ def test_longest_blocks(gpu):
         with O.ninv_mode(O.NINV_DIRECT), O.offset_mode(O.OFFSET_REFERENCE):
             ref = O.apply_weights(x, blocks, LAM, invtt)
         assert np.max(np.abs(out - ref)) <= 1e-12 * np.max(np.abs(ref)), n
+
+
+@pytest.mark.parametrize("gap", [0, 5])
+def test_partials_of_many_chunks(gpu, gap):
+    """more than 8192 chunks of 1024 samples (four a workgroup): blocks that end inside chunks,
+    several in one chunk, a last part chunk and samples past the blocks"""
+    blocks = np.array([3_000_001, 64, 100, 70, 2_000_000, 1023, 3_400_000 + 777], np.int32)
+    m = int(blocks.sum()) + gap
+    rows = {int(n): W.invtt_block(max(int(n), 2 * LAM), LAM, 1.0, 0.2, 1.5) for n in set(blocks)}
+    invtt = np.concatenate([rows[int(n)] for n in blocks])
+    pix = np.repeat(3 * (np.arange(m) % 97), 3).astype(np.int32) + np.tile(np.arange(3, dtype=np.int32), m)
+    x = np.random.default_rng(m).standard_normal(m) + 0.7
+    with gpu.Problem(pix, np.tile([1.0, 0.3, -0.2], m), blocks, LAM, invtt,
+                     opts=gpu.options(offset_mode=gpu.MGPU_OFFSET_REFERENCE)) as pb:
+        out = pb.apply_weights(x)
+    with O.ninv_mode(O.NINV_DIRECT), O.offset_mode(O.OFFSET_REFERENCE):
+        ref = O.apply_weights(x, blocks, LAM, invtt)
+    assert np.max(np.abs(out - ref)) <= 1e-12 * np.max(np.abs(ref))
