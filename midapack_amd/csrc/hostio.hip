@@ -8,10 +8,11 @@
 // pinned buffers (two in flight) and queues the DMA on its own stream, so the
 // host copies of one worker overlap the DMA of the others.  The pool is
 // allocated once per process (hipHostMalloc; freed by mappraiser_gpu_finalize)
-// and used by one transfer at a time (others wait for it).  A staged transfer
-// is complete when the call returns: the caller's stream never waits on the
-// pool's events, which the next transfer (possibly another host thread's)
-// records again as soon as the pool is released.
+// and used by one transfer at a time: while it is taken, copies of caller's
+// arrays go as plain copies beside it and only h2d_staged_fill, which has no other
+// form, waits for it.  A staged transfer is complete when the call returns: the
+// caller's stream never waits on the pool's events, which the next transfer
+// (possibly another host thread's) records again as soon as the pool is released.
 #include "mgpu_internal.h"
 
 #include <algorithm>
@@ -116,11 +117,12 @@ int run_workers(int device, int workers, F fn) {
 }  // namespace
 
 int h2d_staged(int device, void *d, const void *h, size_t bytes, hipStream_t s) {
-    if (bytes < kStageMin) {
+    std::unique_lock<std::mutex> lk(g_pool.busy, std::defer_lock);
+    if (bytes >= kStageMin) lk.try_lock();
+    if (!lk.owns_lock()) {  // small or pool busy: another thread's transfer may hold it for long
         MGPU_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
         return MGPU_OK;
     }
-    std::lock_guard<std::mutex> lk(g_pool.busy);
     MGPU_RET(pool_ready(device));
     const StageSplit sp(bytes, g_pool.workers);
     const int W = sp.workers;
@@ -173,11 +175,11 @@ int h2d_staged_fill(int device, void *d, size_t bytes, const StageProducer &fill
 }
 
 int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t after, const StageConsumer *consume) {
+    MGPU_HIP(hipEventSynchronize(after));  // before the pool is taken; its streams wait on no other stream
     std::unique_lock<std::mutex> lk(g_pool.busy, std::defer_lock);
     if (bytes >= (consume ? kStageWork : kStageMin)) lk.try_lock();
     if (!lk.owns_lock()) {
         // small or pool busy: one copy, then the consumer over the whole array
-        MGPU_HIP(hipEventSynchronize(after));
         if (consume) {
             std::vector<unsigned char> tmp(bytes);
             MGPU_HIP(hipMemcpy(tmp.data(), d, bytes, hipMemcpyDeviceToHost));
@@ -193,7 +195,6 @@ int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t afte
     const size_t nch = sp.n;
     const unsigned char *dd = (const unsigned char *) d;
     unsigned char *hh = (unsigned char *) h;
-    MGPU_HIP(hipEventSynchronize(after));  // the pool's streams wait on no other stream
     return run_workers(device, W, [&](int w) -> int {
         hipStream_t st = g_pool.ws[device][w];
         auto issue = [&](size_t k, int b) -> int {
