@@ -33,6 +33,7 @@ struct Gate {
 Gate held_event;  // its address is the event handle
 const hipEvent_t kHeld = reinterpret_cast<hipEvent_t>(&held_event);
 int dummy;
+std::atomic<int> copies{0};  // device copies made
 }  // namespace
 
 extern "C" {
@@ -41,9 +42,11 @@ hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return *p = malloc(n), hipSuccess; }
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
-hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
+    return copies++, memcpy(d, s, n), hipSuccess;
+}
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
-    return memcpy(d, s, n), hipSuccess;
+    return copies++, memcpy(d, s, n), hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
     return *s = reinterpret_cast<hipStream_t>(&dummy), hipSuccess;
@@ -94,7 +97,7 @@ static bool ends(Gate &gate, F f) {
 int main() {
     const size_t MiB = (size_t) 1 << 20;
     // every kind of transfer with the pool free, at the sizes where its form changes
-    for (size_t n : {MiB * 0 + 12, MiB / 4 - 12, MiB / 4 + 12, 4 * MiB - 12, 4 * MiB, 16 * MiB + 12, 100 * MiB + 24}) {
+    for (size_t n : {MiB * 0 + 12, MiB / 4 - 12, MiB / 4 + 12, 4 * MiB + 12, 8 * MiB - 12, 8 * MiB, 16 * MiB - 12, 16 * MiB + 12, 100 * MiB + 24}) {
         const Bytes src = pattern(n);
         Bytes dst(n), back(n);
         check(h2d_staged(0, dst.data(), src.data(), n, nullptr) == MGPU_OK && dst == src, "upload", n);
@@ -107,6 +110,16 @@ int main() {
         Bytes used(n);
         const StageConsumer take = [&](size_t off, const void *c, size_t len) { memcpy(used.data() + off, c, len); };
         check(d2h_staged(0, nullptr, src.data(), n, nullptr, &take) == MGPU_OK && used == src, "consumed download", n);
+    }
+    // one plain copy up to the sizes where staging is the faster form
+    for (size_t n : {4 * MiB, 8 * MiB - 8, 8 * MiB, 16 * MiB - 8, 16 * MiB}) {
+        const Bytes src = pattern(n);
+        Bytes up(n), down(n);
+        copies = 0;
+        check(h2d_staged(0, up.data(), src.data(), n, nullptr) == MGPU_OK && (copies == 1) == (n < 16 * MiB), "upload's form", n);
+        copies = 0;
+        check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr) == MGPU_OK && (copies == 1) == (n < 8 * MiB),
+              "download's form", n);
     }
     // a transfer that another one holds up goes straight through as a plain copy
     for (size_t n : {MiB, 4 * MiB, 16 * MiB, 64 * MiB}) {
