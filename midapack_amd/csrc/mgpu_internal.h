@@ -110,9 +110,10 @@ bool serving_thread();
 
 // Copies between the caller's pageable host arrays and the device through a
 // process-wide pool of pinned staging buffers (hostio.hip).  h2d_staged: when
-// it returns, the host array may be reused, and work queued on s afterwards
-// sees the data (copies of 16 MiB and more are complete on return if the pool was
-// free; the others are queued on s).  d2h_staged: the copies start once the event `after` has
+// it returns, work queued on s afterwards sees the data and a pageable host array
+// may be reused, a page-locked one once s has reached the copy (pageable copies of
+// 16 MiB and more are complete on return if the pool was free; the others are
+// queued on s).  d2h_staged: the copies start once the event `after` has
 // completed; when it returns the data has been delivered, either copied to h or, with
 // a consumer, handed to consume(offset, chunk, bytes) chunk by chunk (called
 // from several threads at once on disjoint chunks; offsets and all chunks but the

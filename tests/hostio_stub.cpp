@@ -33,13 +33,24 @@ struct Gate {
 Gate held_event;  // its address is the event handle
 const hipEvent_t kHeld = reinterpret_cast<hipEvent_t>(&held_event);
 int dummy;
-std::atomic<int> copies{0};  // device copies made
+std::atomic<int> copies{0};           // device copies made
+const unsigned char *locked = nullptr;  // the page-locked array
+std::atomic<int> last_error{hipSuccess};
 }  // namespace
 
 extern "C" {
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "stub"; }
+hipError_t hipGetLastError() { return (hipError_t) last_error.exchange(hipSuccess); }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+    if (!locked || p != locked) {
+        last_error = hipErrorInvalidValue;
+        return hipErrorInvalidValue;
+    }
+    a->type = hipMemoryTypeHost;
+    return hipSuccess;
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return *p = malloc(n), hipSuccess; }
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
@@ -120,6 +131,21 @@ int main() {
         copies = 0;
         check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr) == MGPU_OK && (copies == 1) == (n < 8 * MiB),
               "download's form", n);
+    }
+    // page-locked arrays are copied directly, and asking about the others leaves no error behind
+    check(last_error == hipSuccess, "no error left", 0);
+    for (size_t n : {16 * MiB, 64 * MiB + 24}) {
+        const Bytes src = pattern(n);
+        Bytes up(n), down(n);
+        copies = 0;
+        locked = src.data();
+        check(h2d_staged(0, up.data(), src.data(), n, nullptr) == MGPU_OK && copies == 1 && up == src,
+              "page-locked upload", n);
+        copies = 0;
+        locked = down.data();
+        check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr) == MGPU_OK && copies == 1 && down == src,
+              "page-locked download", n);
+        locked = nullptr;
     }
     // a transfer that another one holds up goes straight through as a plain copy
     for (size_t n : {MiB, 4 * MiB, 16 * MiB, 64 * MiB}) {
