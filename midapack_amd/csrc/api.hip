@@ -765,7 +765,7 @@ int pcg_gls_impl(const char *outpath, const char *ref, int m, int nnz, int *pix,
             err_dn = "hipSetDevice failed in the side-effect thread";
             return;
         }
-        rc_dn = d2h_staged(dev, nullptr, d_loc, sizeof(int) * mm * 3, e_loc, &apply_side_effects);
+        rc_dn = d2h_staged(dev, nullptr, d_loc, sizeof(int) * mm * 3, e_loc, s, &apply_side_effects);
         if (rc_dn != MGPU_OK) err_dn = mappraiser_gpu_last_error();
     });
     std::vector<double> hist(maxiter > 0 ? maxiter : 1);

@@ -26,7 +26,7 @@ namespace {
 
 constexpr size_t kStageChunk = (size_t) 12 << 20;  // bytes per chunk at most (a whole number of units)
 constexpr size_t kStageUnit = 48 << 10;            // chunks are multiples of it, and so of 8, 12 and 16
-// Plain copies below kStageUp and kStageDown go through hipMemcpyAsync and hipMemcpy;
+// Plain copies below kStageUp and kStageDown go through hipMemcpyAsync;
 // copies with host work on every chunk (packing, side effects) are shared by a
 // thread per kStageWork bytes, two chunks each.  (A drop-in solve of 3.1 M samples,
 // whose 38 MB of local indices and side effects one thread took through a plain
@@ -191,18 +191,24 @@ int h2d_staged_fill(int device, void *d, size_t bytes, const StageProducer &fill
     return MGPU_OK;
 }
 
-int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t after, const StageConsumer *consume) {
-    MGPU_HIP(hipEventSynchronize(after));  // before the pool is taken; its streams wait on no other stream
+int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t after, hipStream_t s,
+               const StageConsumer *consume) {
     std::unique_lock<std::mutex> lk(g_pool.busy, std::defer_lock);
-    if (consume ? bytes >= kStageWork : bytes >= kStageDown && !page_locked(h)) lk.try_lock();
+    if (consume ? bytes >= kStageWork : bytes >= kStageDown && !page_locked(h)) {
+        MGPU_HIP(hipEventSynchronize(after));  // before the pool is taken; its streams wait on no other stream
+        lk.try_lock();
+    }
     if (!lk.owns_lock()) {
-        // small, page-locked or pool busy: one copy, then the consumer over the whole array
+        // small, page-locked or pool busy: one copy, then the consumer over the whole array.
+        // (A map queued on the solve's stream: small solves take 10-20 us less than
+        // with a wait for the event and a blocking copy.)
         if (consume) {
+            MGPU_HIP(hipEventSynchronize(after));
             std::vector<unsigned char> tmp(bytes);
             MGPU_HIP(hipMemcpy(tmp.data(), d, bytes, hipMemcpyDeviceToHost));
             (*consume)(0, tmp.data(), bytes);
         } else {
-            MGPU_HIP(hipMemcpy(h, d, bytes, hipMemcpyDeviceToHost));
+            MGPU_HIP(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, s));
         }
         return MGPU_OK;
     }

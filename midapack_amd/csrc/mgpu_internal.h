@@ -113,11 +113,12 @@ bool serving_thread();
 // it returns, work queued on s afterwards sees the data and a pageable host array
 // may be reused, a page-locked one once s has reached the copy (pageable copies of
 // 16 MiB and more are complete on return if the pool was free; the others are
-// queued on s).  d2h_staged: the copies start once the event `after` has
-// completed; when it returns the data has been delivered, either copied to h or, with
-// a consumer, handed to consume(offset, chunk, bytes) chunk by chunk (called
-// from several threads at once on disjoint chunks; offsets and all chunks but the
-// last are multiples of 48 KiB).
+// queued on s).  d2h_staged: work queued on s has produced the data before the event
+// `after`.  With a consumer they are handed to consume(offset, chunk, bytes) chunk by
+// chunk before the call returns (from several threads at once on disjoint chunks;
+// offsets and all chunks but the last are multiples of 48 KiB); else they are in h when
+// it returns or, for small and page-locked arrays and a busy pool, once s has reached
+// the copy.
 using StageConsumer = std::function<void(size_t off, const void *chunk, size_t bytes)>;
 // h2d_staged_fill: `bytes` of device data produced on the host chunk by chunk:
 // fill(off, chunk, len) writes bytes [off, off + len) of the data into the
@@ -126,8 +127,8 @@ using StageConsumer = std::function<void(size_t off, const void *chunk, size_t b
 using StageProducer = std::function<void(size_t off, void *chunk, size_t bytes)>;
 int h2d_staged_fill(int device, void *d, size_t bytes, const StageProducer &fill);
 int h2d_staged(int device, void *d, const void *h, size_t bytes, hipStream_t s);
-int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t after,
-               const StageConsumer *consume = nullptr);
+int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t after, hipStream_t s,
+               const StageConsumer *consume);
 void staging_free();
 
 // buffers owned by a problem; returned to the cache in its destructor (after

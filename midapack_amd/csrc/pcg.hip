@@ -1021,7 +1021,7 @@ int pcg_run(Problem &pb, const double *d_signal, const double *d_noise, double t
     MGPU_HIP(hipMemcpyAsync(hf, flag, sizeof(hf), hipMemcpyDeviceToHost, s));
     MGPU_HIP(hipMemcpyAsync(hs.data(), S, sizeof(double) * hs.size(), hipMemcpyDeviceToHost, s));
     MGPU_HIP(hipMemcpyAsync(hstate.data(), state, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
-    if (h_x) MGPU_RET(d2h_staged(pb.device, h_x, x, sizeof(double) * n, pb.ev1, nullptr));
+    if (h_x) MGPU_RET(d2h_staged(pb.device, h_x, x, sizeof(double) * n, pb.ev1, s, nullptr));
     MGPU_HIP(hipStreamSynchronize(s));
     if (h_hist) MGPU_HIP(hipMemcpy(h_hist, d_hist, sizeof(double) * (size_t) maxiter * nseg, hipMemcpyDeviceToHost));
     float ms = 0.f;

@@ -36,6 +36,8 @@ int dummy;
 std::atomic<int> copies{0};           // device copies made
 const unsigned char *locked = nullptr;  // the page-locked array
 std::atomic<int> last_error{hipSuccess};
+hipStream_t last_stream = nullptr;      // of the last queued copy
+const hipStream_t kOwn = reinterpret_cast<hipStream_t>(&copies);
 }  // namespace
 
 extern "C" {
@@ -56,7 +58,8 @@ hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
     return copies++, memcpy(d, s, n), hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
+    if (st == kOwn || !last_stream) last_stream = st;
     return copies++, memcpy(d, s, n), hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
@@ -117,10 +120,10 @@ int main() {
             memcpy(c, src.data() + off, len);
         });
         check(rc == MGPU_OK && made == src, "produced upload", n);
-        check(d2h_staged(0, back.data(), src.data(), n, nullptr, nullptr) == MGPU_OK && back == src, "download", n);
+        check(d2h_staged(0, back.data(), src.data(), n, nullptr, nullptr, nullptr) == MGPU_OK && back == src, "download", n);
         Bytes used(n);
         const StageConsumer take = [&](size_t off, const void *c, size_t len) { memcpy(used.data() + off, c, len); };
-        check(d2h_staged(0, nullptr, src.data(), n, nullptr, &take) == MGPU_OK && used == src, "consumed download", n);
+        check(d2h_staged(0, nullptr, src.data(), n, nullptr, nullptr, &take) == MGPU_OK && used == src, "consumed download", n);
     }
     // one plain copy up to the sizes where staging is the faster form
     for (size_t n : {4 * MiB, 8 * MiB - 8, 8 * MiB, 16 * MiB - 8, 16 * MiB}) {
@@ -129,8 +132,18 @@ int main() {
         copies = 0;
         check(h2d_staged(0, up.data(), src.data(), n, nullptr) == MGPU_OK && (copies == 1) == (n < 16 * MiB), "upload's form", n);
         copies = 0;
-        check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr) == MGPU_OK && (copies == 1) == (n < 8 * MiB),
+        check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr, nullptr) == MGPU_OK && (copies == 1) == (n < 8 * MiB),
               "download's form", n);
+    }
+    // a plain download is queued on the caller's stream and waits for nothing else
+    {
+        const Bytes src = pattern(MiB);
+        Bytes down(MiB);
+        last_stream = nullptr;
+        held_event.set(false);
+        check(ends(held_event, [&] { return d2h_staged(0, down.data(), src.data(), MiB, kHeld, kOwn, nullptr); }) &&
+                      last_stream == kOwn && down == src,
+              "download queued on its stream", MiB);
     }
     // page-locked arrays are copied directly, and asking about the others leaves no error behind
     check(last_error == hipSuccess, "no error left", 0);
@@ -143,7 +156,7 @@ int main() {
               "page-locked upload", n);
         copies = 0;
         locked = down.data();
-        check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr) == MGPU_OK && copies == 1 && down == src,
+        check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr, nullptr) == MGPU_OK && copies == 1 && down == src,
               "page-locked download", n);
         locked = nullptr;
     }
@@ -166,14 +179,14 @@ int main() {
               "upload beside a busy pool", n);
         a.join();
         occupy(b);
-        check(ends(gate, [&] { return d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr); }) && down == src,
+        check(ends(gate, [&] { return d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr, nullptr); }) && down == src,
               "download beside a busy pool", n);
         b.join();
         // a download that waits for the device does not hold the pool meanwhile
         Bytes made(n), used(n);
         const StageConsumer take = [&](size_t off, const void *c, size_t len) { memcpy(used.data() + off, c, len); };
         held_event.set(false);
-        std::thread w([&] { d2h_staged(0, nullptr, src.data(), n, kHeld, &take); });
+        std::thread w([&] { d2h_staged(0, nullptr, src.data(), n, kHeld, nullptr, &take); });
         while (!held_event.waiting) std::this_thread::yield();
         check(ends(held_event, [&] {
                   return h2d_staged_fill(0, made.data(), n, [&](size_t off, void *c, size_t len) {
