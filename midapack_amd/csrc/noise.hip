@@ -13,7 +13,8 @@
 //      window = ifftshift(chebwin(2 lambda, 150 dB)) (or the general Gaussian
 //      of utils.py:569-573).
 // The reference fits with scipy's trust-region-reflective least squares; here
-// a bounded Levenberg-Marquardt runs one workgroup per block on the device.
+// a bounded Levenberg-Marquardt runs on the device, one workgroup for a short block
+// and 16 for a step of a long one.
 // Both minimise the same objective; results agree to the fit tolerance.
 //
 // FFTs: batched Stockham passes in HBM, four radix-2 stages a launch in
@@ -371,7 +372,8 @@ constexpr int kFitIter = 400;
 // block), k_fit_step decides and takes the step.  Bound by the logarithms and
 // exponentials (VALU): on 64 blocks of 2^17 samples one workgroup a block, with
 // two model passes an iteration, took 18.4 ms; 64 evaluations of 28 us and
-// decisions of 6 us take 2.2 ms.
+// decisions of 6 us take 2.2 ms.  Short blocks are fitted by a workgroup each
+// (k_fit_block, see kBlockRows).
 struct FitState {
     double p[4], q[4];   // best point, trial point (a, alpha, fknee, fmin)
     double A[13];        // normal equations at p: J^T J (0..9), J^T r (10..12: its last three)
@@ -402,43 +404,36 @@ __global__ void k_fit_init(FitState *__restrict__ st, int nb) {
     F.first = 1;
 }
 
+// (r, dh_alpha, dh_fknee, dh_fmin) of frequency i + 1 at the trial point
+__device__ __forceinline__ void fit_term(int64_t i, double n, double fsamp, const double (&q)[4],
+                                         const double *__restrict__ yb, double *v) {
+    const double f = (double) (i + 1) * fsamp / n;
+    const Model md = model_at(f, q[1], q[2], q[3]);
+    v[0] = q[0] + md.h - yb[i];
+    v[1] = md.dh_alpha;
+    v[2] = md.dh_fknee;
+    v[3] = md.dh_fmin;
+}
+
 __global__ __launch_bounds__(kChainWG) void k_fit_eval(const double *__restrict__ y, const int64_t *__restrict__ yoff,
                                                        const int *__restrict__ nlen, double fsamp,
+                                                       const int *__restrict__ list,
                                                        const FitState *__restrict__ st, double *__restrict__ parts) {
-    const int b = blockIdx.x / kChainGroups, g = blockIdx.x % kChainGroups;
+    const int k = blockIdx.x / kChainGroups, g = blockIdx.x % kChainGroups, b = list[k];
     if (st[b].done) return;
     const int64_t n = nlen[b], K = n / 2;
     const double *yb = y + yoff[b] + 1;
-    const double q0 = st[b].q[0], q1 = st[b].q[1], q2 = st[b].q[2], q3 = st[b].q[3];
+    const double q[4] = {st[b].q[0], st[b].q[1], st[b].q[2], st[b].q[3]};
     chain_sums<4, kFitSums>(
-            K, g,
-            [&](int64_t i, double *v) {
-                const double f = (double) (i + 1) * fsamp / (double) n;
-                const Model md = model_at(f, q1, q2, q3);
-                v[0] = q0 + md.h - yb[i];
-                v[1] = md.dh_alpha;
-                v[2] = md.dh_fknee;
-                v[3] = md.dh_fmin;
-            },
-            fit_pair, parts + (int64_t) b * kFitSums * kChains);
+            K, g, [&](int64_t i, double *v) { fit_term(i, (double) n, fsamp, q, yb, v); }, fit_pair,
+            parts + (int64_t) k * kFitSums * kChains);
 }
 
-// one workgroup per block: sums of the evaluation at q, accept or reject, next
-// trial point; *left counts the blocks that go on
-__global__ __launch_bounds__(64 * kFitSums) void k_fit_step(const double *__restrict__ parts,
-                                                            const int *__restrict__ nlen, FitState *__restrict__ st,
-                                                            int *__restrict__ left) {
-    __shared__ double sh[kFitSums];
-    const int b = blockIdx.x;
-    FitState &F = st[b];
-    if (F.done) return;  // written by this block's thread 0 of an earlier launch only
-    const int wv = threadIdx.x >> 6;
-    const double v = chain_tree(parts + ((int64_t) b * kFitSums + wv) * kChains);
-    if ((threadIdx.x & 63) == 0) sh[wv] = v;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
+// The sums of an evaluation at q, by one thread: accept or reject, then the next
+// trial point or F.done
+__device__ __forceinline__ void fit_decide(FitState &F, const double *sums, int n) {
     const double lo[4] = {-20.0, -10.0, 1e-12, 0.0}, hi[4] = {0.0, 0.0, 20.0, 1.0};
-    const double cq = sh[13];
+    const double cq = sums[13];
     bool accept = false, stop = false;
     if (F.first) {
         F.first = 0;
@@ -460,14 +455,13 @@ __global__ __launch_bounds__(64 * kFitSums) void k_fit_step(const double *__rest
     }
     if (stop) {
         F.done = 1;
-        atomicSub(left, 1);
         return;
     }
     if (accept) {
-        F.A[0] = (double) (nlen[b] / 2);  // the sum of 1 * 1
-        for (int e = 0; e < 9; e++) F.A[1 + e] = sh[e];
-        F.jr0 = sh[9];
-        for (int e = 0; e < 3; e++) F.A[10 + e] = sh[10 + e];
+        F.A[0] = (double) (n / 2);  // the sum of 1 * 1
+        for (int e = 0; e < 9; e++) F.A[1 + e] = sums[e];
+        F.jr0 = sums[9];
+        for (int e = 0; e < 3; e++) F.A[10 + e] = sums[10 + e];
     }
     // damped step (J^T J + mu diag) d = -J^T r, projected on the bounds
     const double mu = F.mu;
@@ -530,6 +524,66 @@ __global__ __launch_bounds__(64 * kFitSums) void k_fit_step(const double *__rest
         pn += p[i] * p[i];
     }
     F.tiny = sqrt(dn) <= 1e-14 * (sqrt(pn) + 1e-14) ? 1 : 0;
+}
+
+// one workgroup per listed block: the chains' trees and the decision; *left counts
+// the blocks that go on
+__global__ __launch_bounds__(64 * kFitSums) void k_fit_step(const double *__restrict__ parts,
+                                                            const int *__restrict__ nlen,
+                                                            const int *__restrict__ list, FitState *__restrict__ st,
+                                                            int *__restrict__ left) {
+    __shared__ double sums[kFitSums];
+    const int b = list[blockIdx.x];
+    FitState &F = st[b];
+    if (F.done) return;  // written by this block's thread 0 of an earlier launch only
+    const int wv = threadIdx.x >> 6;
+    const double v = chain_tree(parts + ((int64_t) blockIdx.x * kFitSums + wv) * kChains);
+    if ((threadIdx.x & 63) == 0) sums[wv] = v;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    fit_decide(F, sums, nlen[b]);
+    if (F.done) atomicSub(left, 1);
+}
+
+// The whole fit of a listed block by one workgroup, a thread a chain: the terms,
+// their order and so the bits are those of k_fit_eval and k_fit_step.
+__global__ __launch_bounds__(kChains) void k_fit_block(const double *__restrict__ y, const int64_t *__restrict__ yoff,
+                                                       const int *__restrict__ nlen, double fsamp,
+                                                       const int *__restrict__ list, FitState *__restrict__ st) {
+    __shared__ double chain[kFitSums][kChains];
+    __shared__ double sums[kFitSums];
+    __shared__ FitState F;
+    const int b = list[blockIdx.x], t = threadIdx.x, n = nlen[b], K = n / 2;
+    const double *__restrict__ yb = y + yoff[b] + 1;
+    if (t == 0) F = st[b];
+    __syncthreads();
+    while (!F.done) {  // kFitIter + 1 evaluations at most
+        const double q[4] = {F.q[0], F.q[1], F.q[2], F.q[3]};
+        double acc[kFitSums];
+#pragma unroll
+        for (int s = 0; s < kFitSums; s++) acc[s] = 0.0;
+        for (int i = t; i < K; i += kChains) {
+            double v[4];
+            fit_term(i, (double) n, fsamp, q, yb, v);
+#pragma unroll
+            for (int s = 0; s < kFitSums; s++) {
+                int ia, ib;
+                fit_pair(s, ia, ib);
+                acc[s] += ib < 0 ? v[ia] : v[ia] * v[ib];
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < kFitSums; s++) chain[s][t] = acc[s];
+        __syncthreads();
+        for (int s = t >> 6; s < kFitSums; s += kChains / 64) {
+            const double v = chain_tree(chain[s]);
+            if ((t & 63) == 0) sums[s] = v;
+        }
+        __syncthreads();
+        if (t == 0) fit_decide(F, sums, n);
+        __syncthreads();
+    }
+    if (t == 0) st[b] = F;
 }
 
 // psdm1 of the fitted model on rfftfreq(n), extended to the full even sequence
@@ -636,6 +690,14 @@ static const std::vector<double> &apod_window(int lambda, int kind) {
     return cache[{lambda, kind}] = w;
 }
 
+// Longest chains of a block that one workgroup fits (n <= 8193).  It runs through
+// them at about 0.5 us a term where k_fit_eval and k_fit_step cost two launches a step,
+// for every block until the last one is done: 4096 blocks of 300 samples 71.6 ms with
+// them and 6.0 with k_fit_block, 256 of 4096 samples 6.0 and 2.9, one of 8192 0.54 and
+// 0.47; with 32 terms (16384 samples) it loses unless the blocks fill the chip (one
+// block 0.51 and 0.71, 256 blocks 5.66 and 5.56), with 256 always (64 blocks 6.0 and 15.6).
+static constexpr int kBlockRows = 16;
+
 int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_sizes, int lambda, double fsamp,
                 int window_kind, double *d_invtt, double *h_params) {
     hipStream_t s = pb.stream;
@@ -656,7 +718,7 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
     for (int b = 0; b < nb; b++) yoff[b + 1] = yoff[b] + block_sizes[b] / 2 + 1;
     double *d_win, *d_y, *d_parts;
     int64_t *d_start, *d_yoff;
-    int *d_len, *d_left;
+    int *d_len, *d_left, *d_list;
     FitState *d_fit;
     MGPU_RET(pb.arena.alloc(&d_win, (size_t) lambda));
     MGPU_RET(pb.arena.alloc(&d_start, (size_t) nb + 1));
@@ -665,8 +727,16 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
     MGPU_RET(pb.arena.alloc(&d_left, 1));
     MGPU_RET(pb.arena.alloc(&d_y, (size_t) yoff[nb]));
     MGPU_RET(pb.arena.alloc(&d_fit, (size_t) nb));
-    const int fit_run = std::min(nb, 1 << 14);  // blocks evaluated by one launch (28 KB of chains each)
-    MGPU_RET(pb.arena.alloc(&d_parts, (size_t) fit_run * kFitSums * kChains));
+    // the blocks that a workgroup each fits, then the others
+    std::vector<int> list((size_t) nb);
+    for (int b = 0; b < nb; b++) list[b] = b;
+    const auto split = std::stable_partition(list.begin(), list.end(),
+                                             [&](int b) { return block_sizes[b] / 2 <= kBlockRows * kChains; });
+    const int nshort = (int) (split - list.begin()), nlong = nb - nshort;
+    const int fit_run = std::min(nlong, 1 << 14);  // blocks evaluated by one launch (28 KB of chains each)
+    MGPU_RET(pb.arena.alloc(&d_list, (size_t) nb));
+    MGPU_RET(pb.arena.alloc(&d_parts, (size_t) std::max(fit_run, 1) * kFitSums * kChains));
+    MGPU_HIP(hipMemcpyAsync(d_list, list.data(), sizeof(int) * nb, hipMemcpyHostToDevice, s));
     MGPU_HIP(hipMemcpyAsync(d_win, win.data(), sizeof(double) * lambda, hipMemcpyHostToDevice, s));
     MGPU_HIP(hipMemcpyAsync(d_start, start.data(), sizeof(int64_t) * (nb + 1), hipMemcpyHostToDevice, s));
     MGPU_HIP(hipMemcpyAsync(d_yoff, yoff.data(), sizeof(int64_t) * (nb + 1), hipMemcpyHostToDevice, s));
@@ -684,18 +754,22 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
         if (pass == 1) {
             k_fit_init<<<grid_for(nb, 256), 256, 0, s>>>(d_fit, nb);
             MGPU_LAUNCHED();
-            int left = nb;
+            if (nshort > 0) {
+                k_fit_block<<<nshort, kChains, 0, s>>>(d_y, d_yoff, d_len, fsamp, d_list, d_fit);
+                MGPU_LAUNCHED();
+            }
+            int left = nlong;
             MGPU_HIP(hipMemcpyAsync(d_left, &left, sizeof(int), hipMemcpyHostToDevice, s));
             // an evaluation and a decision a step, kFitIter of them after the first at
             // most; the host looks every kFitPoll steps whether a block is left
             constexpr int kFitPoll = 8;
             for (int it = 0; it <= kFitIter && left > 0; it++) {
-                for (int b0 = 0; b0 < nb; b0 += fit_run) {
+                for (int b0 = nshort; b0 < nb; b0 += fit_run) {
                     const unsigned n = (unsigned) std::min(fit_run, nb - b0);
-                    k_fit_eval<<<n * kChainGroups, kChainWG, 0, s>>>(d_y, d_yoff + b0, d_len + b0, fsamp, d_fit + b0,
+                    k_fit_eval<<<n * kChainGroups, kChainWG, 0, s>>>(d_y, d_yoff, d_len, fsamp, d_list + b0, d_fit,
                                                                      d_parts);
                     MGPU_LAUNCHED();
-                    k_fit_step<<<n, 64 * kFitSums, 0, s>>>(d_parts, d_len + b0, d_fit + b0, d_left);
+                    k_fit_step<<<n, 64 * kFitSums, 0, s>>>(d_parts, d_len, d_list + b0, d_fit, d_left);
                     MGPU_LAUNCHED();
                 }
                 if (it % kFitPoll == kFitPoll - 1) {
@@ -776,7 +850,7 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
         }
     }
     for (void *p : {(void *) d_win, (void *) d_start, (void *) d_yoff, (void *) d_len, (void *) d_left, (void *) d_y,
-                    (void *) d_fit, (void *) d_parts})
+                    (void *) d_fit, (void *) d_parts, (void *) d_list})
         pb.arena.release(p);
     return MGPU_OK;
 }
