@@ -115,7 +115,6 @@ __global__ void k_blue_prep(const double *__restrict__ x, const int64_t *__restr
     const int64_t b = gid / M, t = gid % M;
     const int64_t n = nlen[b];
     A[gid] = t < n ? cmul(make_double2(x[xoff[b] + t], 0.0), chirp(t, n, -1)) : make_double2(0.0, 0.0);
-    if (!B) return;  // the chirp's spectrum is there already
     double2 v = make_double2(0.0, 0.0);
     if (t < n)
         v = chirp(t, n, +1);
@@ -150,10 +149,9 @@ struct Dft {
     int logm, batch;
     bool pow2;
     int64_t nout_max;
-    double2 *a = nullptr, *b = nullptr, *c = nullptr;  // c: the chirp's spectrum (Bluestein), kept between transforms
+    double2 *a = nullptr, *b = nullptr, *c = nullptr;  // c: the chirp's spectrum (Bluestein)
     double2 *X = nullptr;                              // [batch * stride] the transform
     int64_t stride = 0;
-    bool have_chirp = false;
 
     Dft(Problem &p, int logm_, int batch_, bool pow2_, int64_t nout)
         : pb(p), logm(logm_), batch(batch_), pow2(pow2_), nout_max(nout) {}
@@ -205,11 +203,10 @@ struct Dft {
             stride = M;
             return MGPU_OK;
         }
-        k_blue_prep<<<grid_for(total, 256), 256, 0, s>>>(d_x, d_xoff, d_nlen, logm, batch, a, have_chirp ? nullptr : c);
+        k_blue_prep<<<grid_for(total, 256), 256, 0, s>>>(d_x, d_xoff, d_nlen, logm, batch, a, c);
         MGPU_LAUNCHED();
         MGPU_RET(fft(a, b, -1, nullptr, nullptr));
-        if (!have_chirp) MGPU_RET(fft(c, b, -1, nullptr, nullptr));
-        have_chirp = true;
+        MGPU_RET(fft(c, b, -1, nullptr, nullptr));
         k_pointwise<<<grid_for(total, 256), 256, 0, s>>>(a, c, total);
         MGPU_LAUNCHED();
         MGPU_RET(fft(a, b, +1, nullptr, nullptr));
@@ -807,7 +804,7 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
                 }
                 int *d_blk, *d_nlen;
                 int64_t *d_xoff;
-                double *d_xw, *d_w2, *d_ps;
+                double *d_xw, *d_w2 = nullptr, *d_ps = nullptr;
                 double2 *d_X = nullptr;
                 Dft dft(pb, logm, batch, p2, nmax);
                 MGPU_RET(dft.alloc());
@@ -815,8 +812,10 @@ int noise_invtt(Problem &pb, const double *d_noise, int nb, const int *block_siz
                 MGPU_RET(pb.arena.alloc(&d_nlen, (size_t) batch));
                 MGPU_RET(pb.arena.alloc(&d_xoff, (size_t) batch));
                 MGPU_RET(pb.arena.alloc(&d_xw, (size_t) tot));
-                MGPU_RET(pb.arena.alloc(&d_w2, (size_t) batch));
-                MGPU_RET(pb.arena.alloc(&d_ps, (size_t) 3 * kChains * batch));
+                if (pass == 0) {
+                    MGPU_RET(pb.arena.alloc(&d_w2, (size_t) batch));
+                    MGPU_RET(pb.arena.alloc(&d_ps, (size_t) 3 * kChains * batch));
+                }
                 if (!p2) MGPU_RET(pb.arena.alloc(&d_X, (size_t) tot));
                 MGPU_HIP(hipMemcpyAsync(d_blk, blk.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
                 MGPU_HIP(hipMemcpyAsync(d_nlen, nlen.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
