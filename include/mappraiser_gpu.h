@@ -46,7 +46,10 @@ typedef struct mgpu_options {
                            MGPU_REFRESH_ADAPTIVE: when a segment's FP32-updated residual norm has
                            fallen 10x below its last FP64 value or 64 iterations after it, at
                            the start of the next poll block */
-    int tile_log2;      /* real FFT tile length 2^k of the Toeplitz product; 0 = autotuned choice */
+    int tile_log2;      /* real FFT tile length 2^k of the Toeplitz product; 0 = chosen from the
+                           band, all blocks of that band and the precision, so that the
+                           last bits of a block's product may depend on the other blocks
+                           (not with k > 0) */
     int poll_every;     /* PCG: iterations launched between host convergence polls (default 8) */
     int profile;        /* 1: time every kernel class with HIP events on the handle's stream */
     int offset_mode;    /* per-block offset handling of N^-1 (MGPU_OFFSET_*), default REFERENCE */

@@ -474,10 +474,9 @@ struct TwoLevel {
 // (block c*ndet + j) and span their CES, so every table indexed by a CES
 // sample is shared by the CES's detectors.
 // ---------------------------------------------------------------------------
-struct TItem {           // one workgroup of T^T: a sweep, an azimuth bin or a time bin of a block
-    int b, kind, lo, hi; // block; kind 0 sweep, 1 azimuth bin (range in the azimuth order), 2 time bin
-    int64_t rel;         // first output amplitude, relative to the block's amplitudes
-    int stride, pad;     // distance between the class outputs (sweeps or time bins)
+struct TItem {           // one workgroup of k_tmpl_az: an azimuth bin of a block
+    int b, lo, hi;       // block; the bin's range in the azimuth order
+    int64_t rel;         // its amplitude, relative to the block's
 };
 struct TPieces {         // T^T's pieces of one CES: runs of samples of one sweep (or time bin) inside a chunk
     int p0, h0;          // first sweep piece and first time-bin piece (numbered over all CES)
@@ -606,22 +605,21 @@ int launch_trmatvec(Problem &pb, const double *d_y, double *d_x, const double *d
 int launch_trmatvec_f32(Problem &pb, const float *d_y, double *d_x, const double *d_hvec,
                         double *d_dotpart, int *nparts);
 int trmatvec_nparts(const Problem &pb);
-// smallest valid local pixel of every P chunk (INT32_MAX: none), on the host
 
 // Block definitions and the Toeplitz set-up (defineBlocks_avg, tpltz_init).
 // invtt holds the band of every block, block b's band at the running sum of
 // the earlier blocks' bands (b * lambda when every band is lambda long).
 // block_lambda (optional): the band of each block (default: lambda for all);
-// block_log2n (optional): the FP64 tile length of each block (default: the
-// length choose_log2n picks for its band and longest block of that band).
+// block_log2n (optional): the tile length of each block (default: the length
+// choose_log2n picks for the blocks of its band and the precision).
 int toeplitz_plan(Problem &pb, const int *block_sizes, int nb, int lambda, const double *d_invtt,
                   const double *h_invtt, const int *block_lambda = nullptr, const int *block_log2n = nullptr);
 // N^-1 on d_in (its per-block partials must already be in tp.d_partials unless
 // compute_partials) -> d_out (may not alias d_in)
-// N^-1 (s + n) with white noise in one pass
-int toeplitz_diag_sum(Problem &pb, const double *d_s, const double *d_n, double *d_out);
 int toeplitz_apply(Problem &pb, const double *d_in, double *d_out, bool compute_partials);
 int toeplitz_apply_f32(Problem &pb, const float *d_in, float *d_out, bool compute_partials);
+// N^-1 (s + n) -> d_out with white noise (lambda 1, no block means) in one pass
+int toeplitz_diag_sum(Problem &pb, const double *d_s, const double *d_n, double *d_out);
 // scratch of one N^-1 product: partial sums [nchunks + nb], means [nb], slice
 // sums of the symmetric mode's output mean [nb * 8]
 struct ToeplitzScratch {
@@ -637,7 +635,8 @@ int toeplitz_apply_scratch(Problem &pb, const double *d_in, double *d_out, doubl
 int noalloc_scratch_init(int device);
 int toeplitz_apply_noalloc(Problem &pb, const double *d_in, double *d_out, hipStream_t stream);
 int tile_variant_count(bool fp32, int log2n);
-// real tile length 2^k the plan of a lambda / longest block would use (0: no tiles)
+// log2 of the tile length that a plan of these blocks of one band would use, fp32: for
+// the FP32 products of a mixed solve (0: lambda 1; -1: no length holds the band)
 int toeplitz_tile_log2(int lambda, const int *block_sizes, int nb, bool fp32, int forced);
 const char *tile_variant_desc(bool fp32, int log2n, int variant);
 

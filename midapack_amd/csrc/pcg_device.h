@@ -112,7 +112,7 @@ __device__ __forceinline__ double reduce_parts(const double *__restrict__ p, int
 }
 
 // Largest number of partials of a segment that the map kernels sum themselves
-// (fused_sums): every workgroup then reads them all, four loads a thread and
+// (`fused` of pcg_run): every workgroup then reads them all, four loads a thread and
 // set, which costs about 1 us against 4.3-7.3 us and a launch for a reduction
 // kernel.  A segment of 1024 workgroups is a map of 262144 pixels; with the
 // 4096 of a 1024^2 map the reads (32 KB a set and workgroup) would add more

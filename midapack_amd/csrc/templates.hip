@@ -917,7 +917,7 @@ int templates_build(Problem &pb, const mgpu_templates *t) {
         for (int a = 0; a < M.nsss; a++) {  // bin a occupies a contiguous range of the azimuth order
             int e = k;
             while (e < C.len && C.az[C.perm[0][e]] == a) e++;
-            items.push_back(TItem{b, 1, k, e, (int64_t) M.npoly * C.ns + a, 0, 0});
+            items.push_back(TItem{b, k, e, (int64_t) M.npoly * C.ns + a});
             k = e;
         }
     }

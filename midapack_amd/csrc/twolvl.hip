@@ -572,8 +572,6 @@ int twolvl_build(Problem &pb, const double *d_signal, const double *d_noise) {
     return MGPU_OK;
 }
 
-constexpr int kSumZn = 16, kSumWgs = 512;
-
 int twolvl_apply(Problem &pb, const double *d_g, const double *d_gp, double *d_Cg, double *d_h, double *d_part,
                  bool init, const int *d_state, const int *d_flag) {
     const TwoLevel &T = pb.tl;
@@ -583,9 +581,13 @@ int twolvl_apply(Problem &pb, const double *d_g, const double *d_gp, double *d_C
     MGPU_ARG(T.zn > 0 && T.ld == n, "two-level preconditioner not built for this map");
     k_zt_part<<<dim3(T.nzt, T.zn), kZB, 0, s>>>(T.d_Z, T.ld, n, d_g, T.d_part, T.nzt, T.zt_len, d_state, d_flag);
     MGPU_LAUNCHED();
-    // Every workgroup of the apply reads the zn * nzt partials and Em1 again: less
-    // than a launch while the columns are few and the workgroups about one round of
-    // the chip (8 columns, 256 workgroups: 1 us against 4.7); past that k_zt_fin reads them once.
+    // Every workgroup of the apply reads the zn * nzt partials and Em1 again, which takes
+    // less time than k_zt_fin and its launch (an iteration with 8 columns of 41030 pixels
+    // 52.3 -> 50.3 us, of 82004 72.0 -> 70.3, of 112505 with 16 columns 97.3 -> 95.3).  The
+    // limits are about a round of the chip: past them the same 2 us are 1 to 2 % of an
+    // iteration (164361 pixels, 8 columns: 104.8 and 102.5 us, 32: 175.9 and 172.4) and
+    // with 625781 nothing (16 columns: 378.4 and 378.6), while the reads grow with the workgroups.
+    constexpr int kSumZn = 16, kSumWgs = 512;
     const bool sum = T.zn <= kSumZn && G.nwg <= kSumWgs;
     if (!sum) {
         k_zt_fin<<<1, kZB, 0, s>>>(T.d_part, T.nzt, T.zn, T.d_Em1, T.d_qtx, d_state, d_flag);
