@@ -806,26 +806,31 @@ __global__ __launch_bounds__(kPtBlock) void k_trmatvec(const int64_t *__restrict
         const int width = (int) ((base[s + 1] - b0) / kSlice);
         const int *__restrict__ cte = ct + b0 + lane;
         const TW2 *__restrict__ cwe = cw12 + b0 + lane;
-        // The last step holds what is left, its loads past the width clamped to the
-        // last hit and its terms skipped: with one hit at a time instead, up to 15
-        // latencies of two dependent loads followed (12 small maps in a batch:
-        // 19.0 -> 14.3 us; 32 detectors x 2^18 samples: 52.5 -> 48.0 us; FP32 and
-        // the 64 x 2^20 raster unchanged).  The FP64 kernel with I weights takes 8
-        // at a time there: with 16 it needs 146 registers and loses a quarter of
-        // its waves.
+        // What is left is one step of the next power of two, its loads past the width
+        // clamped to the last hit and its terms skipped: with one hit at a time instead,
+        // up to 15 latencies of two dependent loads followed (12 small maps in a batch:
+        // 19.0 -> 14.3 us; 32 detectors x 2^18 samples: 52.5 -> 48.0 us; the
+        // 64 x 2^20 raster unchanged), and with always a full step a few hits cost the
+        // issue of all its loads (10^6 pixels of 17 hits, scans crossing: one at a time
+        // 144.2 us, a full step 143.5, now 139.7; 31 hits 244.5, 244.6, 238.9.  Where
+        // every sample of a wave lies on another line, fewer loads in flight reuse more
+        // of y in L2: 17 hits 247, 255, 245, 31 hits 408, 501, 456.)  The FP64 kernel with I
+        // weights takes 8 at a time there: with 16 it needs 146 registers and loses a
+        // quarter of its waves.
         constexpr int kSteps = sizeof(TY) == 8 ? 16 : 4, UR = W0 && kSteps == 16 ? 8 : kSteps;
-        auto step = [&](int i, auto rest) {
+        auto step = [&](int i, auto hits, auto rest) {
+            constexpr int U = decltype(hits)::value;
             constexpr bool REST = decltype(rest)::value;
-            constexpr int U = REST ? UR : kSteps;
             int t[U];
             TW2 w[U];
             double yt[U];
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int k = (REST ? min(i + u, width - 1) : i + u) * kSlice;
-                t[u] = cte[k];
-                w[u] = cwe[k];
-            }
+            for (int u = 0; u < U; u++) t[u] = cte[(REST ? min(i + u, width - 1) : i + u) * kSlice];
+            // FP32: the samples' numbers first, since y waits for them and loads return in
+            // order (uneven hits, I weights: 3428 -> 3344 us; FP64 is slower with the fence)
+            if constexpr (sizeof(TY) == 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; u++) w[u] = cwe[(REST ? min(i + u, width - 1) : i + u) * kSlice];
 #pragma unroll
             for (int u = 0; u < U; u++) yt[u] = t[u] >= 0 && (!REST || i + u < width) ? (double) y[t[u]] : 0.0;
 #pragma unroll
@@ -836,9 +841,28 @@ __global__ __launch_bounds__(kPtBlock) void k_trmatvec(const int64_t *__restrict
                 a2 += (double) w[u].y * yt[u];
             }
         };
+        auto at_most = [&](int i, auto hits) { step(i, hits, std::true_type{}); };
         int i = 0;
-        for (; i + kSteps <= width; i += kSteps) step(i, std::false_type{});
-        for (; i < width; i += UR) step(i, std::true_type{});
+        for (; i + kSteps <= width; i += kSteps) step(i, std::integral_constant<int, kSteps>{}, std::false_type{});
+        while (i < width) {
+            const int left = width - i;
+            if (UR > 8 && left > 8) {
+                at_most(i, std::integral_constant<int, 16>{});
+                i += 16;
+            } else if (UR > 4 && left > 4) {
+                at_most(i, std::integral_constant<int, 8>{});
+                i += 8;
+            } else if (left > 2) {
+                at_most(i, std::integral_constant<int, 4>{});
+                i += 4;
+            } else if (left > 1) {
+                at_most(i, std::integral_constant<int, 2>{});
+                i += 2;
+            } else {
+                at_most(i, std::integral_constant<int, 1>{});
+                i += 1;
+            }
+        }
         x[3 * qq] = a0;
         x[3 * qq + 1] = a1;
         x[3 * qq + 2] = a2;
