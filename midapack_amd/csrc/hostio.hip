@@ -26,16 +26,17 @@ namespace {
 
 constexpr size_t kStageChunk = (size_t) 12 << 20;  // bytes per chunk at most (a whole number of units)
 constexpr size_t kStageUnit = 48 << 10;            // chunks are multiples of it, and so of 8, 12 and 16
-// Plain copies below kStageUp and kStageDown go through hipMemcpyAsync;
-// copies with host work on every chunk (packing, side effects) are shared by a
-// thread per kStageWork bytes, two chunks each.  (A drop-in solve of 3.1 M samples,
-// whose 38 MB of local indices and side effects one thread took through a plain
-// copy: 27 -> 11 ms.)  The threads' start costs more than they save below the two
-// limits: a solve with two uploads of 4.8 MB takes 0.71 ms staged and 0.52 plain, of
-// 12 MB 1.05 and 0.93, of 16 MB 1.21 and 1.18, of 24 MB 1.54 and 1.88; one that
-// downloads a map of 5 MB 1.69 and 1.64, of 8.3 MB 2.39 and 2.46, of 13 MB 3.48 and 3.70.
-constexpr size_t kStageUp = (size_t) 16 << 20;
-constexpr size_t kStageDown = (size_t) 8 << 20;
+// Plain copies below kStageMin go through hipMemcpyAsync; copies with host work
+// on every chunk (packing, side effects) are shared by a thread per kStageWork
+// bytes, two chunks each.  (A drop-in solve of 3.1 M samples, whose 38 MB of local
+// indices and side effects one thread took through a plain copy: 27 -> 11 ms.)  The
+// threads' start costs more than they save below it: a solve with two uploads from
+// arrays that change takes 0.64 ms staged and 0.58 plain with 4.8 MB each, 0.73 and
+// 0.71 with 6.4, 0.78 and 0.80 with 8, 0.89 and 1.00 with 10.6, 1.10 and 1.37 with 16
+// (from the same arrays every time 0.66 and 0.51, 0.73 and 0.60, 0.79 and 0.68, 0.93
+// and 0.84, 1.11 and 1.18); one that downloads a map of 5 MB 1.69 and 1.64, of 8.3 MB
+// 2.39 and 2.46, of 13 MB 3.48 and 3.70.
+constexpr size_t kStageMin = (size_t) 8 << 20;
 constexpr size_t kStageWork = (size_t) 256 << 10;
 constexpr int kMaxWorkers = 8;
 constexpr int kMaxDevices = 16;
@@ -135,7 +136,7 @@ int run_workers(int device, int workers, F fn) {
 
 int h2d_staged(int device, void *d, const void *h, size_t bytes, hipStream_t s) {
     std::unique_lock<std::mutex> lk(g_pool.busy, std::defer_lock);
-    if (bytes >= kStageUp && !page_locked(h)) lk.try_lock();
+    if (bytes >= kStageMin && !page_locked(h)) lk.try_lock();
     if (!lk.owns_lock()) {  // small, page-locked or pool busy: another thread's transfer may hold it for long
         MGPU_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
         return MGPU_OK;
@@ -194,7 +195,7 @@ int h2d_staged_fill(int device, void *d, size_t bytes, const StageProducer &fill
 int d2h_staged(int device, void *h, const void *d, size_t bytes, hipEvent_t after, hipStream_t s,
                const StageConsumer *consume) {
     std::unique_lock<std::mutex> lk(g_pool.busy, std::defer_lock);
-    if (consume ? bytes >= kStageWork : bytes >= kStageDown && !page_locked(h)) {
+    if (consume ? bytes >= kStageWork : bytes >= kStageMin && !page_locked(h)) {
         MGPU_HIP(hipEventSynchronize(after));  // before the pool is taken; its streams wait on no other stream
         lk.try_lock();
     }

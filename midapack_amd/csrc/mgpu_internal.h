@@ -112,7 +112,7 @@ bool serving_thread();
 // process-wide pool of pinned staging buffers (hostio.hip).  h2d_staged: when
 // it returns, work queued on s afterwards sees the data and a pageable host array
 // may be reused, a page-locked one once s has reached the copy (pageable copies of
-// 16 MiB and more are complete on return if the pool was free; the others are
+// 8 MiB and more are complete on return if the pool was free; the others are
 // queued on s).  d2h_staged: work queued on s has produced the data before the event
 // `after`.  With a consumer they are handed to consume(offset, chunk, bytes) chunk by
 // chunk before the call returns (from several threads at once on disjoint chunks;

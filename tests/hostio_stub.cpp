@@ -126,11 +126,11 @@ int main() {
         check(d2h_staged(0, nullptr, src.data(), n, nullptr, nullptr, &take) == MGPU_OK && used == src, "consumed download", n);
     }
     // one plain copy up to the sizes where staging is the faster form
-    for (size_t n : {4 * MiB, 8 * MiB - 8, 8 * MiB, 16 * MiB - 8, 16 * MiB}) {
+    for (size_t n : {4 * MiB, 8 * MiB - 8, 8 * MiB, 16 * MiB}) {
         const Bytes src = pattern(n);
         Bytes up(n), down(n);
         copies = 0;
-        check(h2d_staged(0, up.data(), src.data(), n, nullptr) == MGPU_OK && (copies == 1) == (n < 16 * MiB), "upload's form", n);
+        check(h2d_staged(0, up.data(), src.data(), n, nullptr) == MGPU_OK && (copies == 1) == (n < 8 * MiB), "upload's form", n);
         copies = 0;
         check(d2h_staged(0, down.data(), src.data(), n, nullptr, nullptr, nullptr) == MGPU_OK && (copies == 1) == (n < 8 * MiB),
               "download's form", n);
